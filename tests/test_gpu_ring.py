@@ -1,0 +1,87 @@
+"""GPU parity of the few-tile GEMM (ring_gemm_kernel): calls of 33 rows and more (17 where K >= N) whose grid
+is small take it without a flag, with 16, 32 or 64 rows per workgroup.
+
+Bars as for every linear (rel-L2 <= 1e-3 against the oracle, the reference's rounding-budget gate); identity
+inputs with power-of-two scales are bit-exact; two calls agree bit for bit.
+"""
+import numpy as np
+import pytest
+import torch
+
+import lowbit_hip
+from conftest import announce
+from oracle import lowbit_oracle as o
+from test_gpu_linear import check, problem, run, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# (fmt, M, N, K, group, rank, bias): the last stage's 32 / 64 / 96 codes and whole stages, K below a stage and
+# around the ring's depth, rows and columns at the edges of the 16 / 32 / 64-row tiles, scales of 8 and 28 KB,
+# corrections of one to four eights
+CASES = [
+    ('int4', 33, 64, 32, 32, 0, False), ('int4', 48, 65, 64, 64, 0, True), ('int4', 40, 63, 96, 32, 0, False),
+    ('int4', 37, 200, 128, 128, 0, False), ('int4', 64, 129, 160, 32, 0, True), ('nf4', 50, 192, 576, 32, 0, False),
+    ('nf4', 333, 2560, 960, 64, 0, True), ('nf4', 97, 1000, 992, 32, 0, False), ('nf4', 17, 40, 640, 64, 0, False),
+    ('int8', 31, 33, 768, 768, 0, True), ('int8', 100, 700, 896, 64, 0, False), ('int8', 256, 576, 576, 576, 32, False),
+    ('int8', 256, 1536, 576, 576, 32, True), ('int8', 257, 1500, 1504, 1504, 8, False), ('int4', 65, 190, 1056, 32, 24, True),
+    ('nf4', 129, 577, 224, 32, 16, False), ('int4', 48, 14336, 1024, 128, 0, False), ('int4', 500, 320, 2080, 32, 0, True),
+    ('int4', 64, 500, 4096, 32, 0, False), ('int4', 600, 2048, 2048, 2048, 0, False), ('int8', 513, 2040, 2048, 2048, 0, True),
+]
+
+
+@pytest.mark.parametrize('spec', CASES, ids=lambda s: '-'.join(map(str, s)))
+def test_ring_matches_oracle(device, spec):
+    fmt, m, n, k, group, rank, bias = spec
+    announce('ring', spec)
+    p = problem(np.random.default_rng(m * 977 + n + k + group), fmt, m, n, k, group, rank=rank, bias=bias)
+    got = run(p, device)
+    check(p, got, f'ring {spec}')
+    assert np.array_equal(run(p, device), got)
+
+
+def test_ring_fp16_rows(device):
+    """fp16 weights (no scales) against a double product, a ragged last stage included."""
+    announce('ring fp16')
+    rng = np.random.default_rng(3)
+    for m, n, k in ((40, 70, 96), (256, 576, 576), (65, 300, 1536)):
+        x = rng.standard_normal((m, k)).astype(np.float16)
+        w = (rng.standard_normal((n, k)) * 0.02).astype(np.float16)
+        y = lowbit_hip.linear(to_dev(x, device), to_dev(w, device), None, format='fp16', N=n, K=k, group_size=k)
+        assert o.rel_l2(y.cpu().numpy(), x.astype(np.float64) @ w.astype(np.float64).T) <= 1e-3, (m, n, k)
+
+
+@pytest.mark.parametrize('m,n', [(64, 128), (250, 1000)])
+def test_ring_identity_is_bit_exact(device, m, n):
+    k, group = 480, 32
+    announce('ring identity', m, n)
+    rng = np.random.default_rng(16)
+    data = o.pack(rng.integers(0, 16, n * k).astype(np.uint8))
+    scales = (2.0 ** rng.integers(-10, 3, n * (k // group))).astype(np.float16)
+    w = o.dequantize('int4', (n, k), group, data, scales.tobytes())
+    x = np.zeros((m, k), np.float16)
+    cols = rng.integers(0, k, m)
+    x[np.arange(m), cols] = 1.0
+    y = lowbit_hip.linear(to_dev(x, device), to_dev(np.frombuffer(data, np.uint8), device), to_dev(scales, device),
+                          format='int4', N=n, K=k, group_size=group).cpu().numpy()
+    np.testing.assert_array_equal(y, w[:, cols].T)
+
+
+@pytest.mark.parametrize('columns,pitch', [(200, 208), (203, 211)])
+def test_ring_strided_rows_leave_the_rest(device, columns, pitch):
+    """Strided x and y (16-byte rows and odd ones): the columns past N keep their values; a row of infinities
+    and a NaN stay in their rows."""
+    announce('ring strided', columns, pitch)
+    m, k = 70, 352
+    p = problem(np.random.default_rng(5), 'int4', m, columns, k, 32)
+    wide = torch.full((m, k + 16), float('nan'), dtype=torch.float16, device=device)
+    wide[:, :k] = to_dev(p['x'], device)
+    wide[3, 5], wide[9, 351] = float('inf'), float('nan')
+    y = torch.full((m, pitch), 7.0, dtype=torch.float16, device=device)
+    lowbit_hip.linear(wide[:, :k], to_dev(np.frombuffer(p['data'], np.uint8), device),
+                      to_dev(np.frombuffer(p['scales'], np.float16), device), format='int4', N=columns, K=k,
+                      group_size=32, out=y[:, :columns])
+    got = y.cpu().numpy()
+    assert (got[:, columns:] == 7.0).all()
+    assert not np.isfinite(got[3, :columns]).all() and np.isnan(got[9, :columns]).all()
+    rows = [r for r in range(m) if r not in (3, 9)]
+    check(dict(p, x=p['x'][rows], m=len(rows)), got[rows][:, :columns], 'ring strided')

@@ -135,6 +135,32 @@ __device__ __forceinline__ h8 decode8(const u4 &w, int t8, h2 s2, const uint32_t
   return out;
 }
 
+// Natural-order (k ascending) fp16 decode of one dword of codes for LDS staging.
+template <int FMT, bool SCALED>
+__device__ __forceinline__ h8 decode8_natural(uint32_t w0, uint32_t w1, h2 s2, const uint32_t *nf4_table) {
+  h2 p[4];
+  if constexpr (FMT == FMT_INT4) {
+    int4_pairs(w0, p);  // (c0,c2),(c4,c6),(c1,c3),(c5,c7)
+    h2 q0 = {p[0].x, p[2].x}, q1 = {p[0].y, p[2].y}, q2 = {p[1].x, p[3].x}, q3 = {p[1].y, p[3].y};
+    p[0] = q0; p[1] = q1; p[2] = q2; p[3] = q3;
+  } else if constexpr (FMT == FMT_NF4) {
+    p[0] = as_h2(nf4_table[w0 & 0xFFu]);
+    p[1] = as_h2(nf4_table[(w0 >> 8) & 0xFFu]);
+    p[2] = as_h2(nf4_table[(w0 >> 16) & 0xFFu]);
+    p[3] = as_h2(nf4_table[w0 >> 24]);
+  } else {  // INT8: two dwords
+    h2 a[2], b[2];
+    int8_pairs(w0, a);  // (b0,b2),(b1,b3)
+    int8_pairs(w1, b);
+    p[0] = h2{a[0].x, a[1].x}; p[1] = h2{a[0].y, a[1].y};
+    p[2] = h2{b[0].x, b[1].x}; p[3] = h2{b[0].y, b[1].y};
+  }
+  if (SCALED) { p[0] *= s2; p[1] *= s2; p[2] *= s2; p[3] *= s2; }
+  return __builtin_shufflevector(__builtin_shufflevector(p[0], p[1], 0, 1, 2, 3),
+                                 __builtin_shufflevector(p[2], p[3], 0, 1, 2, 3),
+                                 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
 // Raw buffer resource over [base, base + bytes): loads at or beyond `bytes` return zero.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void *base, size_t bytes) {
   const int records = bytes > 0x7FFFFFF0ull ? 0x7FFFFFF0 : (int)bytes;

@@ -15,6 +15,7 @@
 #include "lb_stream.h"
 #include "lb_gemm.h"
 #include "lb_kernels.h"
+#include "lb_ring.h"
 #include "lb_variants.h"
 #include "lb_wide.h"
 
@@ -415,6 +416,40 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
   return best;
 }
 
+#ifndef LB_RING_MAX_TILES
+#define LB_RING_MAX_TILES 544  // ring_gemm_kernel up to this many 64 x 64 tiles (rows of at least 2048 codes)
+#endif
+
+// 16-row tiles per workgroup (1, 2 or 4) with which ring_gemm_kernel takes a PATH_GEMM call, or 0.  It takes
+// grids of one round (256 workgroups of the smallest tile that allows it: the fewer rows a workgroup has, the
+// shorter its stages), any K the fast paths take, ranks of 8 to 32 in whole eights (the correction in the launch).
+// us, gemm4_kernel 64 x 64 / 128 x 128 with split K and its reduction -> ring_gemm_kernel, one box:
+//   INT4 g64   500x320x960 9.5 -> 6.1, 330x2560x960 10.1 -> 7.3, 700x960x2560 19.2 -> 12.1,
+//              256x4096x4096 25.9 -> 18.8, 48x14336x4096 33.8 -> 18.9
+//   NF4 g64    500x960x2560 15.6 -> 11.8, 333x2560x960 10.5 -> 8.4, 64x8192x3072 19.8 -> 13.6
+//   INT8       700x576x1536 11.8 -> 7.2, 256x576x576 with rank 32 21.2 -> 6.1, 100x2569x3136 rank 8 54.0 -> 12.4
+// Past one round: up to two of INT4 / INT8 / fp16 rows of 2048 codes or more (512x4096x4096 37.2 -> 34.2,
+// 1024x2048x2048 27.6 -> 21.0, 600x2048x2048 20.2 -> 19.2; shorter rows 500x2560x960 11.3 -> 12.5, NF4, whose
+// table reads load LDS, 512x4096x4096 38.7 -> 42.2).  Long rows stay on split K where few workgroups would walk
+// them (INT4 40x2048x8192 18.5 -> 20.0) and, for NF4, past 4096 codes (300x2048x8192 32.3 -> 38.6).
+int ring_rt(const lb_linear_args *a) {
+  const int64_t up_ld = a->up_ld == 0 ? a->rank : a->up_ld;
+  if (a->flags & LB_FLAG_FORCE_GEMM) return 0;
+  if (a->rank > 0 && (a->rank > 32 || a->rank % 8 != 0 || !aligned(a->down, 16) || !aligned(a->up, 16) || up_ld % 8 != 0)) return 0;
+  const bool scaled = a->format != LB_FORMAT_FP16 && !(a->format == LB_FORMAT_INT8 && a->group_size == a->K);
+  if (scaled && (!aligned(a->scales, 16) || ring_scale_kb(a->K / a->group_size) == 0)) return 0;
+  // Byte offsets of a tile's rows are 32-bit.
+  if (64 * a->ldx * 2 > INT32_MAX || 64 * a->K * 2 > INT32_MAX) return 0;
+  const int64_t cols = (a->N + 63) / 64;
+  const int64_t t1 = (a->M + 15) / 16 * cols, t2 = (a->M + 31) / 32 * cols, t4 = (a->M + 63) / 64 * cols;
+  if (a->format == LB_FORMAT_NF4 && a->K > 4096) return 0;
+  if (a->K > 4096 && t1 <= 128) return 0;
+  if (t1 <= 256) return 1;
+  if (t2 <= 256 || a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
+  if (t4 <= 256) return 4;
+  return a->format != LB_FORMAT_NF4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES ? 4 : 0;
+}
+
 // Workspace and kernel path of the compact_groups and W8A8 variants.
 Plan make_variant_plan(const lb_linear_args *a, int variant) {
   Plan pl;
@@ -788,6 +823,36 @@ void dense_fp16(int64_t M, int64_t N, int64_t K, const void *w, int64_t ldw, con
   }
 }
 
+// A PATH_GEMM call on ring_gemm_kernel (no workspace: the correction and the whole K run in the launch).
+void launch_ring_linear(const lb_linear_args *a, const LinearParams &p, int rt, hipStream_t s) {
+  RingParams rp{};
+  rp.x = p.x;
+  rp.M = p.M;
+  rp.K = p.K;
+  rp.ldx = p.ldx;
+  rp.G = p.G;
+  rp.group_shift = p.group_shift;
+  rp.per_row = p.per_row;
+  rp.row_bytes = p.code_ld;
+  RingProblem &q = rp.prob[0];
+  q.codes = p.codes;
+  q.scales = p.scales;
+  q.bias = p.bias;
+  q.y = p.y;
+  q.N = p.N;
+  q.ldy = p.ldy;
+  q.vec = aligned(a->y, 16) && a->ldy % 8 == 0;
+  q.rank = (int)a->rank;
+  if (a->rank > 0) {
+    q.down = static_cast<const f16 *>(a->down);
+    q.up = static_cast<const f16 *>(a->up);
+    q.up_ld = (int)(a->up_ld == 0 ? a->rank : a->up_ld);
+  }
+  const int tiles = (p.N + 63) / 64;
+  for (RingProblem &r : rp.prob) r.tiles_end = tiles;
+  launch_ring(rp, (int)a->format, a->format != LB_FORMAT_FP16 && !p.per_row, a->rank > 0, rt, tiles, s);
+}
+
 // W8A8: quantize the activations into the workspace, then the int8 MFMA GEMV / GEMM (or the
 // generic kernel, which quantizes as it reads).
 void launch_w8a8(const lb_linear_args *a, const Plan &pl, LinearParams p, hipStream_t s) {
@@ -1033,6 +1098,10 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
     } else if (a->M > 16) launch_stream_wide(sp, fmt, !p.per_row, s);
     else if (a->M >= LB_STREAM_ROWS_DECODE_MIN_M) launch_stream_rows(sp, fmt, !p.per_row, s);
     else launch_stream(sp, fmt, !p.per_row, stream_group_span(fmt, a->K, a->group_size), s);
+    return launch_status("lb_linear");
+  }
+  if (const int rt = plan.path == PATH_GEMM ? ring_rt(a) : 0) {
+    launch_ring_linear(a, p, rt, s);
     return launch_status("lb_linear");
   }
   uint8_t *ws = static_cast<uint8_t *>(a->workspace);
