@@ -257,6 +257,53 @@ lb_status lb_decode_stack_release(const void *table);
 
 lb_status lb_decode_check(const void *workspace, size_t timeout_offset, void *stream, uint32_t *timeouts);
 
+/* y[m] = fp16(fp16(x[m] * rsqrt(mean(x[m]^2) + eps)) * gamma) for M contiguous rows of K fp16 values
+ * (K a multiple of 8 up to 4096; 16-byte aligned; y may not overlap x): torch_npu_smollm.py:166-168. */
+lb_status lb_rms_rows(const void *x, const void *gamma, void *y, int64_t M, int64_t K, float eps, void *stream);
+
+/*
+ * One decoder layer over batch x seq token rows: each sequence's rows take positions start ..
+ * start + seq - 1, their rotated keys and their values are written to those cache slots, and row i
+ * attends over slots 0 .. start + i (slots below start are the sequence's earlier tokens).  A prefill
+ * is start = 0, a decode step seq = 1.  Seven launches with the staging of lb_decode_layer
+ * (torch_npu_smollm.py:142-193); the counterpart of the reference's prefill and decode graphs of a
+ * layer (:195-340, :506-544) for any batch and length.  Limits: hidden = 64 heads <= 4096,
+ * intermediate a multiple of 32, at most 2016 positions; q, k, v share a format and group, gate and up
+ * share one; int8 per row with ranks 0, 8, .., 32, or int4 / nf4 with power-of-two groups >= 32 (at most
+ * 64 per row) or fp16, without corrections (LB_UNSUPPORTED otherwise).
+ */
+typedef struct lb_layer_projection {
+  uint32_t format;             /* lb_format */
+  uint32_t reserved;
+  int64_t group_size;          /* int8: K; fp16: ignored */
+  int64_t N, K;
+  const void *codes, *scales;  /* as lb_linear_args; 16-byte aligned */
+  int64_t rank;
+  const void *down, *up;       /* V fp16 [rank, K], U fp16 [N, up_ld], 16-byte aligned */
+  int64_t up_ld;               /* a multiple of 8 */
+} lb_layer_projection;
+
+#define LB_LAYER_ROWS_WORKSPACE_BYTES(rows, hidden, intermediate) \
+  ((size_t)(rows) * (4u * (size_t)(hidden) + (size_t)(intermediate)) * 2u)
+
+typedef struct lb_layer_rows_args {
+  uint32_t struct_size;        /* sizeof(lb_layer_rows_args) */
+  uint32_t reserved;
+  int64_t batch, seq, start;
+  int64_t hidden, intermediate, heads, kv_heads, capacity;
+  const void *x;               /* fp16 [batch, seq, hidden] */
+  void *out;                   /* fp16 [batch, seq, hidden]; may not overlap x */
+  const void *norm1, *norm2;   /* fp16 [hidden] */
+  float eps, scale;            /* RMSNorm epsilon, attention score scale (0.125) */
+  lb_layer_projection proj[7]; /* q, k, v, o, gate, up, down */
+  const void *cos, *sin;       /* fp16 [capacity, 64] */
+  void *keys, *values;         /* fp16 [batch, kv_heads, capacity, 64] */
+  void *workspace;             /* LB_LAYER_ROWS_WORKSPACE_BYTES(batch * seq, hidden, intermediate); any contents */
+  size_t workspace_bytes;
+} lb_layer_rows_args;
+
+lb_status lb_layer_rows(const lb_layer_rows_args *args, void *stream);
+
 /*
  * Greedy step: t = first index of the largest logit (NaN logits are never chosen);
  * token[0] = t; if 0 <= position[0] < limit: tokens[position[0]] = t and position[0] += 1;

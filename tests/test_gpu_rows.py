@@ -1,0 +1,116 @@
+"""GPU parity of lb_layer_rows (a SmolLM layer over batch x seq rows in seven launches) and lb_rms_rows, through
+FrozenSmolLayer against its staged CPU reference: rel-L2 <= 1e-2 on outputs, keys and values (the decoder's bar)
+at the edges of the 16-row tiles, for every weight format and correction rank class.
+"""
+import numpy as np
+import pytest
+import torch
+
+import lowbit_hip
+import smollm_random
+from conftest import announce
+from torch_npu_lowbit import quantize_weight
+from torch_npu_lowbit_correction import LowRankCorrection
+from torch_npu_smollm import _SHAPES, FrozenSmolLayer
+
+pytestmark = pytest.mark.gpu
+
+
+def layer(mode, rank=0, capacity=160, protected=(), seed=3):
+    g = torch.Generator().manual_seed(seed)
+    weights = {n: (torch.randn(s, generator=g) * 0.02 if len(s) == 2 else 1 + 0.1 * torch.randn(s, generator=g)).half()
+               for n, s in _SHAPES.items()}
+    packed = corrections = None
+    if rank:
+        packed = {n: quantize_weight(w, format='int8') for n, w in weights.items() if w.ndim == 2}
+        corrections = {n: LowRankCorrection(s, rank, (torch.randn(rank, s[1], generator=g) * 0.01).half().numpy().tobytes(),
+                                            (torch.randn(s[0], rank, generator=g) * 0.01).half().numpy().tobytes())
+                       for n, s in _SHAPES.items() if len(s) == 2 and n not in protected}
+    return FrozenSmolLayer(smollm_random.config(10000.0, 1), weights, mode=mode, packed_weights=packed,
+                           corrections=corrections, capacity=capacity, fp16_projections=protected)
+
+
+def rel(got, want):
+    want = want.double()
+    return float((got.cpu().double() - want).norm() / want.norm())
+
+
+CASES = [('w8a16', 32, 1, 1), ('w8a16', 32, 1, 16), ('w8a16', 8, 3, 17), ('w8a16', 4, 1, 33), ('w8a16', 0, 2, 64),
+         ('w4a16', 0, 1, 15), ('w4a16', 0, 5, 31), ('nf4a16', 0, 1, 77), ('fp16', 0, 2, 130), ('fp16', 0, 1, 3),
+         ('w8a16', 24, 8, 20), ('nf4a16', 0, 4, 120)]
+
+
+@pytest.mark.parametrize('mode,rank,batch,seq', CASES)
+def test_layer_rows_prefill_and_decode(device, mode, rank, batch, seq):
+    """A prefill of seq rows, then three tokens: every row equals the CPU reference of the whole sequence, and a
+    second continuation of the first snapshot gives the same bits (the snapshot was not changed)."""
+    announce('layer rows', mode, rank, batch, seq)
+    lay = layer(mode, rank)
+    assert 'rows' in lay._dev(device)
+    x = torch.randn(batch, seq + 3, 576, generator=torch.Generator().manual_seed(seq)).half()
+    want, trace = lay.reference_cpu(x)
+    with torch.no_grad():
+        out, first = lay.prefill(x[:, :seq].to(device))
+        assert rel(out, want[:, :seq]) <= 1e-2
+        outs, cache = [], first
+        for t in range(3):
+            o, cache = lay.decode(x[:, seq + t:seq + t + 1].to(device), cache)
+            outs.append(o)
+        assert rel(torch.cat(outs, 1), want[:, seq:]) <= 1e-2
+        assert rel(cache.keys[:, :, :seq + 3], trace['keys']) <= 1e-2 and rel(cache.values[:, :, :seq + 3], trace['values']) <= 1e-2
+        assert not cache.keys[:, :, seq + 3:].any() and not cache.values[:, :, seq + 3:].any()
+        again, _ = lay.decode(x[:, seq:seq + 1].to(device), first)
+        assert torch.equal(again, outs[0])
+        assert rel(lay(x.to(device)), want) <= 1e-2
+
+
+def test_layer_rows_do_not_read_past_the_position(device):
+    """Slots past the new token hold NaN and infinities; a strided input row is taken as it is."""
+    announce('layer rows poison')
+    lay = layer('w4a16')
+    x = torch.randn(2, 40, 1152, generator=torch.Generator().manual_seed(1)).half()[..., ::2]
+    with torch.no_grad():
+        _, cache = lay.prefill(x[:, :35].to(device))
+        want, _ = lay.decode(x[:, 35:36].to(device).clone(), cache)
+        cache.keys[:, :, 36:] = float('nan')
+        cache.values[:, :, 36:] = float('inf')
+        got, _ = lay.decode(x.to(device)[:, 35:36], cache)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize('protected,rows', [(('self_attn.o_proj.weight', 'mlp.down_proj.weight'), True),
+                                            (('self_attn.q_proj.weight',), False)])
+def test_layer_rows_and_protected_projections(device, protected, rows):
+    """fp16-protected projections: in lb_layer_rows where q, k, v and gate, up keep one format, staged otherwise."""
+    announce('layer rows protected', protected)
+    lay = layer('w8a16', 32, protected=protected)
+    assert ('rows' in lay._dev(device)) == rows
+    x = torch.randn(1, 20, 576, generator=torch.Generator().manual_seed(2)).half()
+    want, _ = lay.reference_cpu(x)
+    with torch.no_grad():
+        assert rel(lay(x.to(device)), want) <= 1e-2
+
+
+@pytest.mark.parametrize('rows,width', [(1, 576), (5, 8), (3, 4096), (257, 520)])
+def test_rms_rows(device, rows, width):
+    announce('rms rows', rows, width)
+    g = torch.Generator().manual_seed(rows)
+    x, gamma = torch.randn(rows, width, generator=g).half(), torch.randn(width, generator=g).half()
+    f = x.float()
+    want = (f * torch.rsqrt(f.square().mean(-1, keepdim=True) + 1e-5)).half() * gamma
+    got = lowbit_hip.rms_rows(x.to(device), gamma.to(device)).cpu()
+    # one fp16 rounding of the normalised value may fall on the other side of a tie, one of the product follows
+    assert (np.abs(got.float().numpy() - want.float().numpy()) <= 2 ** -9 * np.abs(want.float().numpy()) + 2 ** -24).all()
+
+
+def test_layer_rows_refuses(device):
+    announce('layer rows refuses')
+    lay = layer('w4a16', capacity=8)
+    rows = lay._dev(device)['rows']
+    x = torch.zeros(1, 4, 576, dtype=torch.float16, device=device)
+    both = torch.zeros(2, 1, 3, 8, 64, dtype=torch.float16, device=device)
+    for start in (-1, 5):
+        with pytest.raises(ValueError, match='capacity'):
+            rows.run(x, both[0], both[1], start)
+    with pytest.raises(ValueError, match='overlaps'):
+        rows.run(x, both[0], both[0], 0)

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
   // What a wave reads of its half of a stage (64 codes): lane (j, g) holds k = 16 g .. 16 g + 15 of it, 8 per
   // MFMA, of activation row 16 r + j and weight row 16 wave + j.
   struct Raw {
-    h8 a[2][RT], za[2], zv[2][ZPER > 0 ? ZPER : 1];
+    h8 a[2][RT], zv[2][ZPER > 0 ? ZPER : 1];
     uint32_t w[BITS / 2];
     f16 s;
   } raw[2];
@@ -232,7 +232,6 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
 #pragma unroll
       for (int i = 0; i < ZPER; ++i) {
         const int z = ZT % 4 != 0 ? min(wave * ZPER + i, ZT - 1) : wave * ZPER + i;
-        if (i == 0) f.za[u] = *reinterpret_cast<const h8 *>(a + (z / ZCOLS) * 4096 + a_at[u]);
         f.zv[u][i] = *reinterpret_cast<const h8 *>(b + T::B_BYTES + (z % ZCOLS) * 4096 + a_at[u]);
       }
     }
@@ -247,13 +246,16 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
       else o.b[u] = __builtin_bit_cast(h8, u4{f.w[4 * u], f.w[4 * u + 1], f.w[4 * u + 2], f.w[4 * u + 3]});
     }
   };
+  static_assert(NV == 0 || RT <= 2, "a wave's z tiles take row tile 0 or RT - 1");
+  const bool z_row = NV > 0 && ZT % 4 == 0 && wave * ZPER / ZCOLS > 0;  // (wave-uniform)
   auto multiply = [&](const Raw &f, const Weights &o) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
       for (int r = 0; r < RT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.a[u][r], o.b[u], acc[r], 0, 0, 0);
 #pragma unroll
-      for (int i = 0; i < ZPER; ++i) zacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.za[u], f.zv[u][i], zacc[i], 0, 0, 0);
+      for (int i = 0; i < ZPER; ++i)
+        zacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(RT > 1 && z_row ? f.a[u][RT - 1] : f.a[u][0], f.zv[u][i], zacc[i], 0, 0, 0);
     }
   };
 
@@ -341,7 +343,6 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
         for (int r = 0; r < RT; ++r) f.a[u][r] = g >= 2 ? zero : f.a[u][r];
 #pragma unroll
         for (int i = 0; i < ZPER; ++i) f.zv[u][i] = g >= 2 ? zero : f.zv[u][i];
-        if (ZPER > 0) f.za[u] = g >= 2 ? zero : f.za[u];
       }
     }
     multiply(f, o);

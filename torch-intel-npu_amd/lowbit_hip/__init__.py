@@ -28,7 +28,8 @@ EXPORTS = ('lb_abi_version', 'lb_status_name', 'lb_last_error', 'lb_failed', 'lb
            'lb_workspace_bytes', 'lb_linear', 'lb_linear_noalloc', 'lb_unpack_codes', 'lb_dequantize')
 NOALLOC_SCRATCH_BYTES = 32 << 20   # LB_NOALLOC_SCRATCH_BYTES
 DECODE_EXPORTS = ('lb_fused_linear', 'lb_decode_attention', 'lb_argmax_next', 'lb_head_next', 'lb_decode_layer',
-                  'lb_decode_stack_prepare', 'lb_decode_stack', 'lb_decode_stack_release', 'lb_decode_check')
+                  'lb_decode_stack_prepare', 'lb_decode_stack', 'lb_decode_stack_release', 'lb_decode_check',
+                  'lb_rms_rows', 'lb_layer_rows')
 PROLOGUES = {'none': 0, 'rmsnorm': 1, 'silu_mul': 2}
 MAX_PROBLEMS, MAX_RANK, MAX_FUSED_K = 3, 32, 1536
 def attention_workspace_bytes(heads, capacity):
@@ -156,6 +157,25 @@ class DecodeStackArgs(ctypes.Structure):
                 ('workspace', ctypes.c_void_p), ('workspace_bytes', ctypes.c_size_t)]
 
 
+class LayerProjection(ctypes.Structure):
+    """Mirror of lb_layer_projection."""
+    _fields_ = [('format', ctypes.c_uint32), ('reserved', ctypes.c_uint32), ('group_size', ctypes.c_int64),
+                ('N', ctypes.c_int64), ('K', ctypes.c_int64), ('codes', ctypes.c_void_p), ('scales', ctypes.c_void_p),
+                ('rank', ctypes.c_int64), ('down', ctypes.c_void_p), ('up', ctypes.c_void_p), ('up_ld', ctypes.c_int64)]
+
+
+class LayerRowsArgs(ctypes.Structure):
+    """Mirror of lb_layer_rows_args."""
+    _fields_ = [('struct_size', ctypes.c_uint32), ('reserved', ctypes.c_uint32),
+                ('batch', ctypes.c_int64), ('seq', ctypes.c_int64), ('start', ctypes.c_int64),
+                ('hidden', ctypes.c_int64), ('intermediate', ctypes.c_int64), ('heads', ctypes.c_int64),
+                ('kv_heads', ctypes.c_int64), ('capacity', ctypes.c_int64),
+                ('x', ctypes.c_void_p), ('out', ctypes.c_void_p), ('norm1', ctypes.c_void_p), ('norm2', ctypes.c_void_p),
+                ('eps', ctypes.c_float), ('scale', ctypes.c_float), ('proj', LayerProjection * 7),
+                ('cos', ctypes.c_void_p), ('sin', ctypes.c_void_p), ('keys', ctypes.c_void_p), ('values', ctypes.c_void_p),
+                ('workspace', ctypes.c_void_p), ('workspace_bytes', ctypes.c_size_t)]
+
+
 _lib = None
 
 
@@ -209,6 +229,11 @@ def library():
         lib.lb_head_next.argtypes = [ctypes.POINTER(FusedLinearArgs), ctypes.c_void_p, ctypes.c_void_p,
                                      ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
                                      ctypes.c_void_p]
+        lib.lb_rms_rows.restype = ctypes.c_int
+        lib.lb_rms_rows.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
+                                    ctypes.c_float, ctypes.c_void_p]
+        lib.lb_layer_rows.restype = ctypes.c_int
+        lib.lb_layer_rows.argtypes = [ctypes.POINTER(LayerRowsArgs), ctypes.c_void_p]
         if lib.lb_abi_version() != ABI_VERSION:
             raise RuntimeError(f'liblowbit_hip ABI {lib.lb_abi_version()} != expected {ABI_VERSION}')
         _lib = lib
@@ -817,3 +842,81 @@ class PreparedStack(_Prepared):
     def counters(self):
         """(workgroups counted over all calls so far, timeout word) of the workspace."""
         return [int(self.workspace[:8].view(torch.int64)), int(self.workspace[8:12].view(torch.int32))]
+
+
+# ---------------------------------------------------------------- several token rows
+def rms_rows(x, gamma, eps=1e-5):
+    """lb_rms_rows: fp16(fp16(x * rsqrt(mean(x^2) + eps)) * gamma) of the contiguous fp16 rows of x [..., K]."""
+    rows, width = x.numel() // x.shape[-1], x.shape[-1]
+    _row(x, 'x', rows * width)
+    _row(gamma, 'gamma', width)
+    y = torch.empty_like(x)
+    _check(library().lb_rms_rows(_ptr(x), _ptr(gamma), _ptr(y), rows, width, eps, _stream(x.device)), 'lb_rms_rows')
+    return y
+
+
+class LayerRows:
+    """lb_layer_rows of one layer's weights: run() takes the rows, the cache and the first position.
+
+    projections: seven dicts (q, k, v, o, gate, up, down) with codes, scales (None for fp16), format, group, N, K
+    and optionally down [rank, K] and up [N, rank].  Holds references to every weight it points at; the rows'
+    buffers belong to each call, so one instance may be used from several streams and threads.
+    """
+
+    MAX_POSITIONS, MAX_GROUPS = 2016, 64
+
+    def __init__(self, projections, *, hidden, intermediate, norm1, norm2, eps, heads, kv_heads, cos, sin, scale=0.125):
+        a = LayerRowsArgs()
+        a.struct_size = ctypes.sizeof(LayerRowsArgs)
+        a.hidden, a.intermediate, a.heads, a.kv_heads = hidden, intermediate, heads, kv_heads
+        a.eps, a.scale, a.capacity = eps, scale, cos.shape[0]
+        keep = [_row(norm1, 'norm1', hidden), _row(norm2, 'norm2', hidden), _row(cos, 'cos', a.capacity * 64),
+                _row(sin, 'sin', a.capacity * 64)]
+        a.norm1, a.norm2, a.cos, a.sin = (_ptr(t) for t in keep)
+        for q, pr in zip(a.proj, projections):
+            q.format, q.group_size, q.N, q.K = FORMATS[pr['format']], pr['group'], pr['N'], pr['K']
+            q.codes, q.scales = _ptr(pr['codes']), _ptr(pr.get('scales'))
+            keep += [pr['codes'], pr.get('scales')]
+            down, up = pr.get('down'), pr.get('up')
+            if down is not None:
+                rank = (down.shape[0] + 7) // 8 * 8
+                if rank != down.shape[0] or up.stride(-1) != 1 or up.stride(0) % 8:  # whole eights: zero ranks add nothing
+                    down = torch.cat((down, down.new_zeros(rank - down.shape[0], down.shape[1])))
+                    up = torch.cat((up, up.new_zeros(up.shape[0], rank - up.shape[1])), 1)
+                down = down.contiguous()
+                q.rank, q.down, q.up, q.up_ld = rank, _ptr(down), _ptr(up), up.stride(0)
+                keep += [down, up]
+        self._template, self._keep, self._device = a, keep, norm1.device
+        self._fn = library().lb_layer_rows
+
+    @classmethod
+    def takes(cls, projections, capacity):
+        """Whether lb_layer_rows takes these projections (its limits, include/lowbit_decode_hip.h)."""
+        kind = [(pr['format'], 0 if pr['format'] == 'fp16' else pr['group']) for pr in projections]
+        if capacity > cls.MAX_POSITIONS or len({kind[0], kind[1], kind[2]}) > 1 or kind[4] != kind[5]:
+            return False
+        for pr in projections:
+            group, width = pr['group'], pr['K']
+            if pr['format'] in ('int4', 'nf4') and (width // group > cls.MAX_GROUPS or not (
+                    group == width or (group >= 32 and group & (group - 1) == 0))):
+                return False
+            if pr['format'] == 'int8' and group != width:
+                return False
+            if pr.get('rank', 0) > MAX_RANK or (pr.get('rank', 0) and pr['format'] != 'int8'):
+                return False
+        return True
+
+    def run(self, x, keys, values, start):
+        """x fp16 [batch, seq, hidden] (contiguous) -> the layer's output; keys and values [batch, kv_heads,
+        capacity, 64] receive slots start .. start + seq - 1."""
+        a = LayerRowsArgs.from_buffer_copy(self._template)
+        a.batch, a.seq, a.start, a.capacity = x.shape[0], x.shape[1], start, keys.shape[2]
+        rows = x.shape[0] * x.shape[1]
+        out = torch.empty_like(x)
+        workspace = torch.empty(rows * (4 * a.hidden + a.intermediate), dtype=torch.float16, device=x.device)
+        a.x, a.out, a.keys, a.values = x.data_ptr(), out.data_ptr(), keys.data_ptr(), values.data_ptr()
+        a.workspace, a.workspace_bytes = workspace.data_ptr(), 2 * workspace.numel()
+        status = self._fn(ctypes.byref(a), _stream(x.device))
+        if status != OK:
+            _check(status, 'lb_layer_rows')
+        return out

@@ -5,9 +5,11 @@ SmolKVCache and FrozenSmolStack keep their constructor arguments (config, weight
 {fp16, w8a16, w4a16, nf4a16}, packed_weights, fp16_projections, corrections), their
 forward / prefill / decode / reference_cpu methods and their fp16 staging (reference
 :142-193).  The reference compiles each layer into one NPU graph; here every projection is
-an lb_linear call of liblowbit_hip (W8 per-row, INT4/NF4 group-32, optional rank-r
-correction) and the glue (RMSNorm, RoPE, attention, SiLU) is staged PyTorch-ROCm ops with
-the same fp16 rounding points.
+low-bit (W8 per-row, INT4/NF4 group-32, optional rank-r correction) and a layer runs as one
+lb_layer_rows call of liblowbit_hip (RMSNorm, projections, RoPE and KV append, attention, SiLU
+and residuals in seven launches, the same fp16 rounding points), for a prefill as for a decode
+step.  Layers it does not take (projections of mixed formats, capacities past 2016) run one lb_linear
+per projection with the glue as staged PyTorch-ROCm ops.
 
 Deviations (the reference limits come from its NPU graph and are lifted):
   * rope_theta: any positive value from the config (the reference accepts only 1e5, :81);
@@ -39,6 +41,9 @@ _SHAPES = {'self_attn.q_proj.weight': (576, 576), 'self_attn.k_proj.weight': (19
            'mlp.gate_proj.weight': (1536, 576), 'mlp.up_proj.weight': (1536, 576),
            'mlp.down_proj.weight': (576, 1536), 'input_layernorm.weight': (576,),
            'post_attention_layernorm.weight': (576,)}
+# Projection order of lb_layer_rows.
+_ROWS_ORDER = ('self_attn.q_proj.weight', 'self_attn.k_proj.weight', 'self_attn.v_proj.weight',
+               'self_attn.o_proj.weight', 'mlp.gate_proj.weight', 'mlp.up_proj.weight', 'mlp.down_proj.weight')
 _REQUIRED = dict(model_type='llama', hidden_size=576, intermediate_size=1536, num_attention_heads=9,
                  num_key_value_heads=3, hidden_act='silu', attention_bias=False, mlp_bias=False,
                  rms_norm_eps=1e-5, rope_scaling=None, pretraining_tp=1)
@@ -75,10 +80,12 @@ def _rope_tables(theta, positions):
 
 
 class _KVStorage:
-    """Device K/V slots shared by the snapshots of one sequence; `high` is the written length."""
+    """Device K/V slots shared by the snapshots of one sequence; `high` is the written length.
+    keys and values are the halves of one tensor, so a copy is one launch."""
 
-    def __init__(self, keys, values, high):
-        self.keys, self.values, self.high = keys, values, high
+    def __init__(self, both, high):
+        self.both, self.high = both, high
+        self.keys, self.values = both[0], both[1]
 
 
 @dataclass(frozen=True, eq=False)
@@ -278,6 +285,11 @@ class FrozenSmolLayer(torch.nn.Module):
                 else:
                     entry = dict(codes=self._weights[name].to(device), scales=None, format='fp16', group=k, N=n, K=k)
                 state['lin'][name] = entry
+            projections = [dict(state['lin'][name]) for name in _ROWS_ORDER]
+            if lowbit_hip.LayerRows.takes(projections, self._capacity):
+                state['rows'] = lowbit_hip.LayerRows(projections, hidden=HIDDEN, intermediate=1536, norm1=state['norm1'],
+                                                     norm2=state['norm2'], eps=1e-5, heads=HEADS, kv_heads=KV_HEADS,
+                                                     cos=state['cos'], sin=state['sin'])
             self._device[key] = state
         return self._device[key]
 
@@ -326,10 +338,13 @@ class FrozenSmolLayer(torch.nn.Module):
         delta = self._linear(state, hidden, 'mlp.down_proj.weight').view(b, s, d)
         return (value + delta).half()
 
-    def _full(self, x):
-        """Causal full-sequence layer on device; returns (out, keys [B,3,S,64], values)."""
+    def _full(self, x, both):
+        """Causal full-sequence layer on device; keys and values go to slots 0 .. S - 1 of
+        both [2, B, 3, slots, 64]."""
         state = self._dev(x.device)
         b, s, d = x.shape
+        if 'rows' in state:
+            return state['rows'].run(x.detach().contiguous(), both[0], both[1], 0)
         n1 = self._norm(x, state['norm1']).view(b * s, d)
         q = self._linear(state, n1, 'self_attn.q_proj.weight').view(b, s, HEADS, HEAD_DIM).transpose(1, 2)
         k = self._linear(state, n1, 'self_attn.k_proj.weight').view(b, s, KV_HEADS, HEAD_DIM).transpose(1, 2)
@@ -340,23 +355,21 @@ class FrozenSmolLayer(torch.nn.Module):
         att = self._attend(q, k, v, mask).transpose(1, 2).reshape(b * s, d)
         delta = self._linear(state, att, 'self_attn.o_proj.weight').view(b, s, d)
         value = (x + delta).half()
-        return self._mlp(state, value), k, v
+        both[0, :, :, :s] = k
+        both[1, :, :, :s] = v
+        return self._mlp(state, value)
 
     def forward(self, x):
-        self._validate_input(x)
-        return self._full(x)[0]
+        b, s, _ = self._validate_input(x)
+        return self._full(x, torch.empty((2, b, KV_HEADS, s, HEAD_DIM), dtype=torch.float16, device=x.device))
 
     def prefill(self, x):
         """Full prefix; returns the output and a KV snapshot (reference :506-523)."""
         b, s, _ = self._validate_input(x)
-        out, k, v = self._full(x)
-        keys = torch.zeros((b, KV_HEADS, self._capacity, HEAD_DIM), dtype=torch.float16, device=x.device)
-        values = torch.zeros_like(keys)
-        keys[:, :, :s] = k
-        values[:, :, :s] = v
-        storage = _KVStorage(keys, values, s)
-        position = torch.tensor([s], dtype=torch.int32, device=x.device)
-        return out, SmolKVCache(self._cache_owner, object(), keys, values, s, position, storage)
+        storage = _KVStorage(torch.zeros((2, b, KV_HEADS, self._capacity, HEAD_DIM), dtype=torch.float16, device=x.device), s)
+        out = self._full(x, storage.both)
+        position = torch.full((1,), s, dtype=torch.int32, device=x.device)
+        return out, SmolKVCache(self._cache_owner, object(), storage.keys, storage.values, s, position, storage)
 
     def _validate_cache(self, x, cache):
         if x.shape[1] != 1 or type(cache) is not SmolKVCache or cache._owner is not self._cache_owner:
@@ -374,9 +387,14 @@ class FrozenSmolLayer(torch.nn.Module):
         state = self._dev(x.device)
         storage = cache._storage
         if storage.high != cache.length:  # decoding from an older snapshot: copy on write
-            storage = _KVStorage(cache.keys.clone(), cache.values.clone(), cache.length)
+            storage = _KVStorage(storage.both.clone(), cache.length)
         p = cache.length
         b = x.shape[0]
+        if 'rows' in state:
+            out = state['rows'].run(x.detach().contiguous(), storage.keys, storage.values, p)
+            storage.high = p + 1
+            position = torch.full((1,), p + 1, dtype=torch.int32, device=x.device)
+            return out, SmolKVCache(self._cache_owner, cache._sequence, storage.keys, storage.values, p + 1, position, storage)
         n1 = self._norm(x, state['norm1']).view(b, HIDDEN)
         q = self._linear(state, n1, 'self_attn.q_proj.weight').view(b, 1, HEADS, HEAD_DIM).transpose(1, 2)
         k = self._linear(state, n1, 'self_attn.k_proj.weight').view(b, 1, KV_HEADS, HEAD_DIM).transpose(1, 2)
@@ -391,7 +409,7 @@ class FrozenSmolLayer(torch.nn.Module):
         delta = self._linear(state, att.transpose(1, 2).reshape(b, HIDDEN), 'self_attn.o_proj.weight').view(b, 1, HIDDEN)
         value = (x + delta).half()
         out = self._mlp(state, value)
-        position = torch.tensor([p + 1], dtype=torch.int32, device=x.device)
+        position = torch.full((1,), p + 1, dtype=torch.int32, device=x.device)
         return out, SmolKVCache(self._cache_owner, cache._sequence, storage.keys, storage.values, p + 1, position,
                                 storage)
 

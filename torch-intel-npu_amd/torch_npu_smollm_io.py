@@ -90,7 +90,8 @@ class FrozenSmolIO(torch.nn.Module):
                 or any(size <= 0 for size in hidden.shape)):
             raise ValueError('Output head requires nonempty FP16 (B,S,576) hidden states')
         self._check(hidden.device)
-        normalized = self.normalize(hidden)
+        normalized = (self.normalize(hidden) if hidden.device.type == 'cpu'
+                      else lowbit_hip.rms_rows(hidden.detach().contiguous(), self.norm))
         b, s, _ = hidden.shape
         if self.head is not None:
             return self._quantized_logits(normalized.reshape(b * s, 576)).view(b, s, self.vocab_size)
