@@ -260,13 +260,23 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(LinearParams p, int 
     }
 }
 
-// Sums split-K partials in a fixed order (deterministic) and applies the epilogue.
+// Sums split-K partials in a fixed order (deterministic) and applies the epilogue; grid (N / 256, M).  Bound by
+// the latency of its loads, so eight slices' partials are requested before the first is added (one at a time,
+// with a 64-bit division for the row: 24x4096 over 16 slices 6.5 us, now 2.9).
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(LinearParams p) {
-  const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (size_t)p.M * p.N) return;
-  const int m = (int)(idx / p.N), n = (int)(idx % p.N);
+  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (n >= p.N) return;
+  const size_t slice = (size_t)p.M * p.N;
+  const float *at = p.partial + (size_t)m * p.N + n;
   float s = 0.0f;
-  for (int sp = 0; sp < p.splits; ++sp) s += p.partial[((size_t)sp * p.M + m) * p.N + n];
+  for (int sp = 0; sp < p.splits; sp += 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = at[(size_t)min(sp + i, p.splits - 1) * slice];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (sp + i < p.splits) s += v[i];
+  }
   store_output(p, m, n, s);
 }
 

@@ -683,6 +683,10 @@ lb_status validate(const lb_linear_args *a, bool check_workspace, Plan *plan) {
   return ok();
 }
 
+void launch_reduce(const LinearParams &p, hipStream_t s) {
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((p.N + 255) / 256), (unsigned)p.M), dim3(256), 0, s, p);
+}
+
 template <int FMT, int MT, int KG, bool SCALED>
 void launch_gemv_t(const LinearParams &p, int kc, hipStream_t s) {
   constexpr int rows = 16 * (kGemvWaves / KG);
@@ -726,8 +730,7 @@ void launch_gemv(int fmt, bool scaled, const LinearParams &p, int kg, int kc, hi
     default: launch_gemv_m<FMT_FP16, false>(p, kg, kc, s); break;
   }
   if (p.splits > 1) {
-    const size_t count = (size_t)p.M * p.N;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, p);
+    launch_reduce(p, s);
   }
 }
 
@@ -774,8 +777,7 @@ void launch_gemm(int fmt, bool scaled, const LinearParams &p, hipStream_t s) {
     default: launch_gemm_t<FMT_FP16, false>(p, s); break;
   }
   if (p.splits > 1) {
-    const size_t count = (size_t)p.M * p.N;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, p);
+    launch_reduce(p, s);
   }
 }
 
@@ -1059,8 +1061,7 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
     if (plan.splits > 1 && !in_kernel) {  // partials [slice, M, N] -> y in slice order (per-row scale, bias)
       p.partial = wp.partial;
       p.splits = plan.splits;
-      const size_t count = (size_t)p.M * p.N;
-      hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, p);
+      launch_reduce(p, s);
     }
     return launch_status("lb_linear");
   }
@@ -1092,8 +1093,7 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
       if (plan.splits > 1 && !in_kernel) {  // partials [slice, M, N] -> y in slice order (per-row scale, bias)
         p.partial = sp.partial;
         p.splits = plan.splits;
-        const size_t count = (size_t)p.M * p.N;
-        hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, p);
+        launch_reduce(p, s);
       }
     } else if (a->M > 16) launch_stream_wide(sp, fmt, !p.per_row, s);
     else if (a->M >= LB_STREAM_ROWS_DECODE_MIN_M) launch_stream_rows(sp, fmt, !p.per_row, s);
