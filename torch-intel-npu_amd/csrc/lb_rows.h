@@ -57,7 +57,8 @@ struct AttendParams {
 // 0 .. start + m, with the staging of the reference (scores fp16(q.k), fp16(* scale), softmax in fp32 rounded to
 // fp16, fp16(P.V)).  Four waves deal the key tiles of Q.K^T (v_mfma_f32_16x16x32_f16, K rows straight from the
 // cache as B operands), all scores of the rows stay in LDS as fp16 (16 x 2016 take 64 KB), each wave normalises
-// four rows there, and P.V is dealt by output columns: wave w owns 16 of the 64 dims.  Rows past the last visible
+// four rows there, sixteen lanes a row, and P.V is dealt by output columns: wave w owns 16 of the 64 dims, its
+// first 256 keys of V requested with the first keys.  Rows past the last visible
 // slot are out of the buffers' range and read zero, so what lies there does not matter.  A whole score row is
 // kept, not folded online, because the reference rounds the normalised probabilities.  Bound by latency at these
 // sizes: 9 heads x 256 rows are 144 workgroups of at most 16 key tiles.
@@ -80,8 +81,19 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendParams p) {
     fq[0] = *reinterpret_cast<const h8 *>(qrow);
     fq[1] = *reinterpret_cast<const h8 *>(qrow + 32);
   }
+  // V of 32 keys as a B operand: lane (j, g) holds dim 16 wave + j of keys 8 g .. 8 g + 7.
+  constexpr int VT = 8;                           // chunks of 32 keys in flight, requested ahead of the scores
+  auto load_v = [&](int c) {
+    h8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = __builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(
+          vbuf, (32 * c + 8 * g + e) * 128 + (16 * wave + j) * 2, 0, 0));
+    return v;
+  };
   const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int KT = 4;                           // key tiles of a wave in flight
+  h8 fv[VT];
   for (int t0 = wave; t0 < tiles; t0 += 4 * KT) {
     h8 fk[KT][2];
 #pragma unroll
@@ -90,6 +102,10 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendParams p) {
       for (int u = 0; u < 2; ++u)
         fk[i][u] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(
             kbuf, (16 * (t0 + 4 * i) + j) * 128 + 64 * u + 16 * g, 0, 0));
+    if (t0 == wave) {
+#pragma unroll
+      for (int i = 0; i < VT; ++i) fv[i] = load_v(i);
+    }
 #pragma unroll
     for (int i = 0; i < KT; ++i) {
       const int t = t0 + 4 * i;
@@ -104,32 +120,61 @@ __global__ __launch_bounds__(256) void attend_rows_kernel(AttendParams p) {
       }
     }
   }
+  if (wave >= tiles) {                            // two key tiles: waves 2 and 3 had none
+#pragma unroll
+    for (int i = 0; i < VT; ++i) fv[i] = load_v(i);
+  }
   __syncthreads();
+  // Softmax: sixteen lanes per row, eight scores a lane at a time; the exponentials of the first 256 scores
+  // stay in registers for the division.
+  {
+    const int r = 4 * wave + (lane >> 4), chunks = 2 * tiles;
+    f16 *row = scores + r * p.pitch + 8 * (lane & 15);
+    constexpr int HELD = 2;
+    float e[HELD][8], top = -INFINITY, total = 0.0f;
+    for (int c = lane & 15, at = 0; c < chunks; c += 16, at += 128) {
+      const h8 v = *reinterpret_cast<const h8 *>(row + at);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = 4 * wave + i;
-    if (r >= rows) break;
-    f16 *row = scores + r * p.pitch;
-    float top = -INFINITY, total = 0.0f;
-    for (int k = lane; k < 16 * tiles; k += 64) top = fmaxf(top, (float)row[k]);
+      for (int q = 0; q < 8; ++q) top = fmaxf(top, (float)v[q]);
+    }
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d));
-    for (int k = lane; k < 16 * tiles; k += 64) total += expf((float)row[k] - top);
+    for (int d = 8; d > 0; d >>= 1) top = fmaxf(top, __shfl_xor(top, d));
 #pragma unroll
-    for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d);
-    for (int k = lane; k < 16 * tiles; k += 64) row[k] = (f16)(expf((float)row[k] - top) / total);
+    for (int i = 0; i < HELD; ++i)
+      if ((lane & 15) + 16 * i < chunks) {
+        const h8 v = *reinterpret_cast<const h8 *>(row + 128 * i);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) total += e[i][q] = expf((float)v[q] - top);
+      }
+    for (int c = (lane & 15) + 16 * HELD, at = 128 * HELD; c < chunks; c += 16, at += 128) {
+      const h8 v = *reinterpret_cast<const h8 *>(row + at);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) total += expf((float)v[q] - top);
+    }
+#pragma unroll
+    for (int d = 8; d > 0; d >>= 1) total += __shfl_xor(total, d);
+#pragma unroll
+    for (int i = 0; i < HELD; ++i)
+      if ((lane & 15) + 16 * i < chunks) {
+        h8 v;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = (f16)(e[i][q] / total);
+        *reinterpret_cast<h8 *>(row + 128 * i) = v;
+      }
+    for (int c = (lane & 15) + 16 * HELD, at = 128 * HELD; c < chunks; c += 16, at += 128) {
+      h8 v = *reinterpret_cast<const h8 *>(row + at);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = (f16)(expf((float)v[q] - top) / total);
+      *reinterpret_cast<h8 *>(row + at) = v;
+    }
   }
   __syncthreads();
   f4 acc = zero;
-  constexpr int VT = 4;                           // chunks of 32 keys in flight
   for (int c0 = 0; c0 < tiles / 2; c0 += VT) {
-    h8 fv[VT];
+    if (c0 > 0) {
 #pragma unroll
-    for (int i = 0; i < VT; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        fv[i][e] = __builtin_bit_cast(f16, __builtin_amdgcn_raw_buffer_load_b16(
-            vbuf, (32 * (c0 + i) + 8 * g + e) * 128 + (16 * wave + j) * 2, 0, 0));
+      for (int i = 0; i < VT; ++i) fv[i] = load_v(c0 + i);
+    }
 #pragma unroll
     for (int i = 0; i < VT; ++i) {
       if (c0 + i >= tiles / 2) break;
