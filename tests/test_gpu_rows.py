@@ -2,6 +2,8 @@
 FrozenSmolLayer against its staged CPU reference: rel-L2 <= 1e-2 on outputs, keys and values (the decoder's bar)
 at the edges of the 16-row tiles, for every weight format and correction rank class.
 """
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,7 @@ import torch
 import lowbit_hip
 import smollm_random
 from conftest import announce
-from torch_npu_lowbit import quantize_weight
+from torch_npu_lowbit import QuantizedLinear, quantize_weight
 from torch_npu_lowbit_correction import LowRankCorrection
 from torch_npu_smollm import _SHAPES, FrozenSmolLayer
 
@@ -101,6 +103,18 @@ def test_rms_rows(device, rows, width):
     got = lowbit_hip.rms_rows(x.to(device), gamma.to(device)).cpu()
     # one fp16 rounding of the normalised value may fall on the other side of a tie, one of the product follows
     assert (np.abs(got.float().numpy() - want.float().numpy()) <= 2 ** -9 * np.abs(want.float().numpy()) + 2 ** -24).all()
+
+
+def test_copies_of_used_modules(device):
+    """Deep copies of a layer and a module that ran bind their own device state and give the same bits."""
+    announce('copies')
+    lay = layer('w8a16', 8)
+    mod = QuantizedLinear(quantize_weight(torch.randn(64, 96) * 0.02, format='int4', group_size=32), bias=torch.randn(64))
+    x, row = torch.randn(1, 5, 576).half().to(device), torch.randn(7, 192).half().to(device)[:, ::2]
+    with torch.no_grad():
+        for a, arg in ((lay, x), (mod, row)):
+            want = a(arg)
+            assert torch.equal(copy.deepcopy(a)(arg), want) and torch.equal(a(arg.contiguous()), want)
 
 
 def test_layer_rows_refuses(device):

@@ -246,6 +246,7 @@ class QuantizedLinear(torch.nn.Module):
         else:
             self._bias = None
         self._bias_device = {}
+        self._bound = {}
 
     @property
     def weight(self):
@@ -270,6 +271,10 @@ class QuantizedLinear(torch.nn.Module):
         return cls(quantize_weight(module.weight, format=format, group_size=group_size), bias=module.bias,
                    compact_groups=compact_groups, activation_scale=activation_scale)
 
+    def __getstate__(self):
+        """Copies and pickles bind their own device calls (those hold raw pointers)."""
+        return {**self.__dict__, '_bound': {}}
+
     def _device_bias(self, device):
         if self._bias is None:
             return None
@@ -282,10 +287,13 @@ class QuantizedLinear(torch.nn.Module):
         """y = x . W^T (+ bias) in fp16 (reference :339-360).  compact_groups selects the per-group
         fp16 products and balanced add tree of the reference's compact graph (:235-256);
         activation_scale selects W8A8 (:224-231), int8 activations on that power-of-two grid."""
-        n, k = self._weight.shape
-        _validate_activation(x, k)
-        codes, scales = self._weight.device_tensors(x.device)
-        flags = lowbit_hip.FLAG_COMPACT_GROUPS if self._compact_groups else 0
-        return lowbit_hip.linear(x, codes, scales, format=self._weight.format, N=n, K=k,
-                                 group_size=self._weight.group_size, bias=self._device_bias(x.device),
-                                 flags=flags, activation_scale=self._activation_scale)
+        _validate_activation(x, self._weight.shape[1])
+        call = self._bound.get(x.device)
+        if call is None:
+            n, k = self._weight.shape
+            codes, scales = self._weight.device_tensors(x.device)
+            flags = lowbit_hip.FLAG_COMPACT_GROUPS if self._compact_groups else 0
+            call = self._bound[x.device] = lowbit_hip.BoundLinear(
+                codes, scales, format=self._weight.format, N=n, K=k, group_size=self._weight.group_size,
+                bias=self._device_bias(x.device), flags=flags, activation_scale=self._activation_scale)
+        return call(x)

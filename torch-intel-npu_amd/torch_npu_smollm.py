@@ -168,6 +168,10 @@ class FrozenSmolLayer(torch.nn.Module):
         return cls(config, weights, mode=mode, packed_weights=packed_weights, fp16_projections=fp16_projections,
                    corrections=corrections, capacity=capacity)
 
+    def __getstate__(self):
+        """Copies and pickles place their own device state (it holds raw pointers to this layer's weights)."""
+        return {**self.__dict__, '_device': {}}
+
     @property
     def mode(self):
         return self._mode
