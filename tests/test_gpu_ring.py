@@ -26,6 +26,11 @@ CASES = [
     ('int8', 256, 1536, 576, 576, 32, True), ('int8', 257, 1500, 1504, 1504, 8, False), ('int4', 65, 190, 1056, 32, 24, True),
     ('nf4', 129, 577, 224, 32, 16, False), ('int4', 48, 14336, 1024, 128, 0, False), ('int4', 500, 320, 2080, 32, 0, True),
     ('int4', 64, 500, 4096, 32, 0, False), ('int4', 600, 2048, 2048, 2048, 0, False), ('int8', 513, 2040, 2048, 2048, 0, True),
+    # up to 32 rows: short rows, many columns, large weights, and every row count class of a correction
+    ('int8', 17, 1536, 576, 576, 0, True), ('int8', 32, 4100, 2304, 2304, 0, False), ('int4', 31, 576, 1536, 64, 0, False),
+    ('int4', 20, 4160, 2560, 32, 0, True), ('nf4', 20, 8190, 256, 128, 0, False), ('int4', 9, 11072, 4096, 128, 0, False),
+    ('int8', 2, 100, 96, 96, 8, True), ('int8', 16, 577, 640, 640, 32, False), ('int8', 19, 64, 4096, 4096, 16, False),
+    ('int4', 5, 130, 320, 64, 24, True), ('nf4', 32, 70, 96, 32, 32, False),
 ]
 
 

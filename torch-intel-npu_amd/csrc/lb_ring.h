@@ -15,6 +15,9 @@
 //     So weights are moved in row order and take their MFMA order from LDS, and scales are not loaded in the loop;
 //   - a step that reads LDS, decodes and multiplies one after the other.  Here the reads of stage t + 2, the
 //     decode of stage t + 1 and the products of stage t are independent of one another.
+// Scales.  A wave's half stage of 64 codes lies in one group when groups are whole multiples of 64 (POST): codes
+// enter the MFMA exact, from a zero accumulator, and the half's sums are scaled into the fp32 accumulator, so
+// the product is the exact x.(q s).  Groups of 32 scale the weights (fp16(q s)) as they are decoded.
 #pragma once
 #include <type_traits>
 #include <utility>
@@ -86,9 +89,10 @@ template <int BYTES> __device__ __forceinline__ int ring_swz(int r) {
   return BYTES == 256 ? r & 15 : BYTES == 128 ? (r >> 1) & 7 : (r >> 2) & 3;
 }
 
-template <int FMT, int SCALE_KB, bool RANKED, int RT, int MODE>
+template <int FMT, int SCALE_KB, bool POST, bool RANKED, int RT, int MODE>
 __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
   constexpr bool PAIR = MODE == RING_SILU, SCALED = SCALE_KB > 0;
+  static_assert(!POST || SCALED, "scales to apply");
   constexpr int NP = PAIR ? 2 : 1;                     // problems a tile's weight rows come from (32 of each)
   constexpr int NV = RANKED ? NP : 0;
   using T = RingTraits<FMT, RT, NV, SCALE_KB>;
@@ -236,26 +240,36 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
       }
     }
   };
-  struct Weights { h8 b[2]; } wt[2];
+  struct Weights { h8 b[2]; float s; } wt[2];
   auto decode = [&](const Raw &f, Weights &o) {
-    const h2 s2 = SCALED ? h2{f.s, f.s} : h2{(f16)1.0f, (f16)1.0f};
+    constexpr bool PRE = SCALED && !POST;
+    const h2 s2 = PRE ? h2{f.s, f.s} : h2{(f16)1.0f, (f16)1.0f};
+    if constexpr (POST) o.s = (float)f.s;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      if constexpr (BITS == 4) o.b[u] = decode8_natural<FMT, SCALED>(f.w[u], 0u, s2, nf4_table);
-      else if constexpr (BITS == 8) o.b[u] = decode8_natural<FMT, SCALED>(f.w[2 * u], f.w[2 * u + 1], s2, nf4_table);
+      if constexpr (BITS == 4) o.b[u] = decode8_natural<FMT, PRE>(f.w[u], 0u, s2, nf4_table);
+      else if constexpr (BITS == 8) o.b[u] = decode8_natural<FMT, PRE>(f.w[2 * u], f.w[2 * u + 1], s2, nf4_table);
       else o.b[u] = __builtin_bit_cast(h8, u4{f.w[4 * u], f.w[4 * u + 1], f.w[4 * u + 2], f.w[4 * u + 3]});
     }
   };
   static_assert(NV == 0 || RT <= 2, "a wave's z tiles take row tile 0 or RT - 1");
   const bool z_row = NV > 0 && ZT % 4 == 0 && wave * ZPER / ZCOLS > 0;  // (wave-uniform)
   auto multiply = [&](const Raw &f, const Weights &o) {
+    f4 part[RT];  // D layout: a lane's sums are all of weight row 16 wave + j, whose scale it holds
+#pragma unroll
+    for (int r = 0; r < RT; ++r) part[r] = POST ? f4{0.0f, 0.0f, 0.0f, 0.0f} : acc[r];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
-      for (int r = 0; r < RT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.a[u][r], o.b[u], acc[r], 0, 0, 0);
+      for (int r = 0; r < RT; ++r) part[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f.a[u][r], o.b[u], part[r], 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < ZPER; ++i)
         zacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(RT > 1 && z_row ? f.a[u][RT - 1] : f.a[u][0], f.zv[u][i], zacc[i], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      if constexpr (POST) acc[r] += o.s * part[r];
+      else acc[r] = part[r];
     }
   };
 

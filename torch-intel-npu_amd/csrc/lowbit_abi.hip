@@ -420,7 +420,12 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 #define LB_RING_MAX_TILES 544  // ring_gemm_kernel up to this many 64 x 64 tiles (rows of at least 2048 codes)
 #endif
 
-// 16-row tiles per workgroup (1, 2 or 4) with which ring_gemm_kernel takes a PATH_GEMM call, or 0.  It takes
+#ifndef LB_RING_MID_CODES
+#define LB_RING_MID_CODES 45000000ll  // 9..16 rows: ring_gemm_kernel from this many codes on
+#endif
+
+// 16-row tiles per workgroup (1, 2 or 4) with which ring_gemm_kernel takes a call, or 0 (the plan, its
+// workspace included, stays what it is: the kernel needs none).  Of the PATH_GEMM calls it takes
 // grids of one round (256 workgroups of the smallest tile that allows it: the fewer rows a workgroup has, the
 // shorter its stages), any K the fast paths take, ranks of 8 to 32 in whole eights (the correction in the launch).
 // us, gemm4_kernel 64 x 64 / 128 x 128 with split K and its reduction -> ring_gemm_kernel, one box:
@@ -432,18 +437,39 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 // 1024x2048x2048 27.6 -> 21.0, 600x2048x2048 20.2 -> 19.2; shorter rows 500x2560x960 11.3 -> 12.5, NF4, whose
 // table reads load LDS, 512x4096x4096 38.7 -> 42.2).  Long rows stay on split K where few workgroups would walk
 // them (INT4 40x2048x8192 18.5 -> 20.0) and, for NF4, past 4096 codes (300x2048x8192 32.3 -> 38.6).
-int ring_rt(const lb_linear_args *a) {
+// Of the calls of up to 32 rows: 17 and more over short rows or enough columns (wide_rows / tile_rows -> ring:
+// INT8 24x14336x4096 24.4 -> 17.9, 32x8192x2048 13.0 -> 8.6, 17x1536x576 4.8 -> 4.1, INT4 32x11008x4096 20.6 -> 13.4,
+// 32x576x1536 7.5 -> 6.0, NF4 32x8192x3072 16.1 -> 10.9; but 24x1024x4096 8.8 -> 9.9, NF4 32x4096x4096 12.5 -> 14.3),
+// 9 to 16 over large weights (INT4 16x11008x4096 16.7 -> 11.9, NF4 12x11008x4096 20.7 -> 15.1; INT4 16x8192x3072
+// 8.7 -> 9.1), not where wide_rows_kernel adds its 4-bit K slices itself, and every call with a correction (no z
+// launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7).
+bool ring_takes(const lb_linear_args *a) {
   const int64_t up_ld = a->up_ld == 0 ? a->rank : a->up_ld;
-  if (a->flags & LB_FLAG_FORCE_GEMM) return 0;
-  if (a->rank > 0 && (a->rank > 32 || a->rank % 8 != 0 || !aligned(a->down, 16) || !aligned(a->up, 16) || up_ld % 8 != 0)) return 0;
+  if (a->rank > 0 && (a->rank > 32 || a->rank % 8 != 0 || !aligned(a->down, 16) || !aligned(a->up, 16) || up_ld % 8 != 0)) return false;
   const bool scaled = a->format != LB_FORMAT_FP16 && !(a->format == LB_FORMAT_INT8 && a->group_size == a->K);
-  if (scaled && (!aligned(a->scales, 16) || ring_scale_kb(a->K / a->group_size) == 0)) return 0;
+  if (scaled && (!aligned(a->scales, 16) || ring_scale_kb(a->K / a->group_size) == 0)) return false;
+  // Groups of 32, powers of two from 64 on, or one per row: a half stage of 64 codes never spans two but for 32.
   // Byte offsets of a tile's rows are 32-bit.
-  if (64 * a->ldx * 2 > INT32_MAX || 64 * a->K * 2 > INT32_MAX) return 0;
+  return 64 * a->ldx * 2 <= INT32_MAX && 64 * a->K * 2 <= INT32_MAX;
+}
+
+int ring_rt(const lb_linear_args *a, const Plan &pl) {
+  constexpr uint32_t kForce =
+      LB_FLAG_FORCE_GEMV | LB_FLAG_FORCE_GEMM | LB_FLAG_FORCE_GENERIC | LB_FLAG_FORCE_STREAM | LB_FLAG_FORCE_WIDE;
+  if ((a->flags & kForce) || pl.path == PATH_GENERIC || pl.path == PATH_ROW || pl.path == PATH_STREAM || !ring_takes(a)) return 0;
   const int64_t cols = (a->N + 63) / 64;
   const int64_t t1 = (a->M + 15) / 16 * cols, t2 = (a->M + 31) / 32 * cols, t4 = (a->M + 63) / 64 * cols;
-  if (a->format == LB_FORMAT_NF4 && a->K > 4096) return 0;
-  if (a->K > 4096 && t1 <= 128) return 0;
+  if (pl.path != PATH_GEMM) {
+    if (a->K > 4096 || a->format == LB_FORMAT_FP16) return 0;
+    const bool nf4 = a->format == LB_FORMAT_NF4, bits8 = a->format == LB_FORMAT_INT8;
+    if (pl.path == PATH_WIDE && !bits8 && pl.splits <= LB_WIDE_IN_KERNEL_SLICES) return 0;
+    const bool few = a->M >= 17 ? (nf4 ? cols >= 128 : a->K <= 2048 || cols >= 64)
+                                : a->M >= 9 && a->N * a->K >= LB_RING_MID_CODES;
+    if (!few && a->rank == 0) return 0;
+  } else {
+    if (a->format == LB_FORMAT_NF4 && a->K > 4096) return 0;
+    if (a->K > 4096 && t1 <= 128) return 0;
+  }
   if (t1 <= 256) return 1;
   if (t2 <= 256 || a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
   if (t4 <= 256) return 4;
@@ -1034,6 +1060,10 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
     launch_fused(fp, fmt, scaled, a->rank > 0, tiles, s);
     return launch_status("lb_linear");
   }
+  if (const int rt = ring_rt(a, plan)) {
+    launch_ring_linear(a, p, rt, s);
+    return launch_status("lb_linear");
+  }
   if (plan.path == PATH_WIDE) {
     WideParams wp{};
     wp.x = p.x;
@@ -1098,10 +1128,6 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
     } else if (a->M > 16) launch_stream_wide(sp, fmt, !p.per_row, s);
     else if (a->M >= LB_STREAM_ROWS_DECODE_MIN_M) launch_stream_rows(sp, fmt, !p.per_row, s);
     else launch_stream(sp, fmt, !p.per_row, stream_group_span(fmt, a->K, a->group_size), s);
-    return launch_status("lb_linear");
-  }
-  if (const int rt = plan.path == PATH_GEMM ? ring_rt(a) : 0) {
-    launch_ring_linear(a, p, rt, s);
     return launch_status("lb_linear");
   }
   uint8_t *ws = static_cast<uint8_t *>(a->workspace);

@@ -13,14 +13,14 @@ using namespace lb::abi;
 
 namespace {
 
-template <int FMT, int SCALE_KB, bool RANKED, int MODE>
+template <int FMT, int SCALE_KB, bool POST, bool RANKED, int MODE>
 void launch_mode_t(const RingParams &p, int rt, int tiles, hipStream_t s) {
   const dim3 grid((unsigned)tiles, (unsigned)((p.M + 16 * rt - 1) / (16 * rt)));
   switch (rt) {
-    case 1: hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, RANKED, 1, MODE>), grid, dim3(kRingThreads), 0, s, p); break;
-    case 2: hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, RANKED, 2, MODE>), grid, dim3(kRingThreads), 0, s, p); break;
+    case 1: hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, POST, RANKED, 1, MODE>), grid, dim3(kRingThreads), 0, s, p); break;
+    case 2: hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, POST, RANKED, 2, MODE>), grid, dim3(kRingThreads), 0, s, p); break;
     default:
-      if constexpr (!RANKED) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, RANKED, 4, MODE>), grid, dim3(kRingThreads), 0, s, p);
+      if constexpr (!RANKED) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, POST, RANKED, 4, MODE>), grid, dim3(kRingThreads), 0, s, p);
       break;
   }
 }
@@ -28,10 +28,16 @@ void launch_mode_t(const RingParams &p, int rt, int tiles, hipStream_t s) {
 template <int MODE>
 void launch_mode(const RingParams &p, int format, bool ranked, int rt, int tiles, hipStream_t s) {
   switch (format) {
-    case FMT_INT8: ranked ? launch_mode_t<FMT_INT8, 0, true, MODE>(p, rt, tiles, s) : launch_mode_t<FMT_INT8, 0, false, MODE>(p, rt, tiles, s); break;
-    case FMT_INT4: launch_mode_t<FMT_INT4, 8, false, MODE>(p, rt, tiles, s); break;
-    case FMT_NF4: launch_mode_t<FMT_NF4, 8, false, MODE>(p, rt, tiles, s); break;
-    default: launch_mode_t<FMT_FP16, 0, false, MODE>(p, rt, tiles, s); break;
+    case FMT_INT8:
+      ranked ? launch_mode_t<FMT_INT8, 0, false, true, MODE>(p, rt, tiles, s) : launch_mode_t<FMT_INT8, 0, false, false, MODE>(p, rt, tiles, s);
+      break;
+    case FMT_INT4:
+      p.group_shift == 5 ? launch_mode_t<FMT_INT4, 8, false, false, MODE>(p, rt, tiles, s) : launch_mode_t<FMT_INT4, 8, true, false, MODE>(p, rt, tiles, s);
+      break;
+    case FMT_NF4:
+      p.group_shift == 5 ? launch_mode_t<FMT_NF4, 8, false, false, MODE>(p, rt, tiles, s) : launch_mode_t<FMT_NF4, 8, true, false, MODE>(p, rt, tiles, s);
+      break;
+    default: launch_mode_t<FMT_FP16, 0, false, false, MODE>(p, rt, tiles, s); break;
   }
 }
 
