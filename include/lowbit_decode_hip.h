@@ -265,7 +265,7 @@ lb_status lb_rms_rows(const void *x, const void *gamma, void *y, int64_t M, int6
  * One decoder layer over batch x seq token rows: each sequence's rows take positions start ..
  * start + seq - 1, their rotated keys and their values are written to those cache slots, and row i
  * attends over slots 0 .. start + i (slots below start are the sequence's earlier tokens).  A prefill
- * is start = 0, a decode step seq = 1.  Seven launches with the staging of lb_decode_layer
+ * is start = 0, a decode step seq = 1.  Seven launches (five for one row in all) with the staging of lb_decode_layer
  * (torch_npu_smollm.py:142-193); the counterpart of the reference's prefill and decode graphs of a
  * layer (:195-340, :506-544) for any batch and length.  Limits: hidden = 64 heads <= 4096,
  * intermediate a multiple of 32, at most 2016 positions; q, k, v share a format and group, gate and up
@@ -284,7 +284,7 @@ typedef struct lb_layer_projection {
 } lb_layer_projection;
 
 #define LB_LAYER_ROWS_WORKSPACE_BYTES(rows, hidden, intermediate) \
-  ((size_t)(rows) * (4u * (size_t)(hidden) + (size_t)(intermediate)) * 2u)
+  (((size_t)(rows) * (4u * (size_t)(hidden) + (size_t)(intermediate)) + 2u * (size_t)(hidden) + (size_t)(intermediate)) * 2u)
 
 typedef struct lb_layer_rows_args {
   uint32_t struct_size;        /* sizeof(lb_layer_rows_args) */

@@ -672,6 +672,11 @@ void launch_stream(const StreamParams &p, int format, bool scaled, int ns, hipSt
   else launch_stream_f<FMT_INT8, false>(p, ns, s);
 }
 
+void launch_decode_attention(const AttnParams &p, hipStream_t s) {
+  hipLaunchKernelGGL(decode_attention_kernel, dim3((unsigned)p.heads, kAttnDimSlices), dim3(256),
+                     (size_t)p.capacity * sizeof(float), s, p);
+}
+
 void launch_fused(const FusedParams &p, int format, bool scaled, bool ranked, int tiles, hipStream_t s) {
   switch (format) {
     case FMT_INT8:
@@ -773,9 +778,7 @@ lb_status lb_decode_attention(const lb_decode_attention_args *a, void *stream) {
                        (size_t)a->capacity * sizeof(float), static_cast<hipStream_t>(stream), p);
     return launch_status("lb_decode_attention");
   }
-  hipLaunchKernelGGL(decode_attention_kernel, dim3((unsigned)a->heads, kAttnDimSlices), dim3(256),
-                     (size_t)a->capacity * sizeof(float),
-                     static_cast<hipStream_t>(stream), p);
+  launch_decode_attention(p, static_cast<hipStream_t>(stream));
   return launch_status("lb_decode_attention");
 }
 

@@ -86,7 +86,27 @@ inline bool stream_rows_ok(int format, long long M, long long K, long long group
   return span == 1;
 }
 
+// One-row attention over the KV cache (decode_attention_kernel, split_attention_kernel).
+struct AttnParams {
+  const f16 *q, *k, *v;      // new rows: q [heads, 64], k and v [kv_heads, 64]
+  const f16 *cos, *sin;      // [capacity, 64]
+  const int64_t *position;   // device scalar: the slot of the new token; null: `slot`
+  f16 *keys, *values;        // [kv_heads, capacity, 64]
+  f16 *out;                  // [heads, 64]
+  int heads, kv_heads, capacity;
+  float scale;
+  // Split form (split_attention_kernel): tagged score words [heads][chunks * 16], then `passed`
+  // (u64) and a timeout word; score workgroups first.
+  uint64_t *words;
+  int chunks;                // position chunks of kAttnChunk per KV head
+  int score_wgs;             // kv_heads * chunks
+  int slot;                  // decode_attention_kernel without a position
+};
+
 // Launches fused_gemv_kernel for `tiles` 16-row tiles (defined with the kernels).
 void launch_fused(const FusedParams &p, int format, bool scaled, bool ranked, int tiles, hipStream_t stream);
+
+// Launches decode_attention_kernel (defined with the kernels).
+void launch_decode_attention(const AttnParams &p, hipStream_t stream);
 
 }  // namespace lb

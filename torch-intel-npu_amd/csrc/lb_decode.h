@@ -772,21 +772,6 @@ __global__ __launch_bounds__(256) void rows_gemv_kernel(const uint8_t *pre_codes
   }
 }
 
-struct AttnParams {
-  const f16 *q, *k, *v;      // new rows: q [heads, 64], k and v [kv_heads, 64]
-  const f16 *cos, *sin;      // [capacity, 64]
-  const int64_t *position;   // device scalar: the slot of the new token
-  f16 *keys, *values;        // [kv_heads, capacity, 64]
-  f16 *out;                  // [heads, 64]
-  int heads, kv_heads, capacity;
-  float scale;
-  // Split form (split_attention_kernel): tagged score words [heads][chunks * 16], then `passed`
-  // (u64) and a timeout word; score workgroups first.
-  uint64_t *words;
-  int chunks;                // position chunks of kAttnChunk per KV head
-  int score_wgs;             // kv_heads * chunks
-};
-
 constexpr int kHeadDim = 64;
 #ifndef LB_ATTN_SLICES
 #define LB_ATTN_SLICES 4
@@ -851,7 +836,7 @@ __global__ __launch_bounds__(256) void decode_attention_kernel(AttnParams p) {
   const int d0 = (int)blockIdx.y * kSliceDims;  // first output dim of this workgroup
   const int group = p.heads / p.kv_heads;
   const int kvh = h / group;
-  const int pos = (int)p.position[0];
+  const int pos = p.position ? (int)p.position[0] : p.slot;
   if (pos < 0 || pos >= p.capacity) {
     // No slot for the new row: nothing is read from or written to the cache, and the
     // workgroup's output dims are NaN, so a caller past the capacity sees it in the result.

@@ -966,7 +966,7 @@ class LayerRows:
         a.batch, a.seq, a.start, a.capacity = x.shape[0], x.shape[1], start, keys.shape[2]
         rows = x.shape[0] * x.shape[1]
         out = torch.empty_like(x)
-        workspace = torch.empty(rows * (4 * a.hidden + a.intermediate), dtype=torch.float16, device=x.device)
+        workspace = torch.empty((rows + 1) * (4 * a.hidden + a.intermediate), dtype=torch.float16, device=x.device)
         a.x, a.out, a.keys, a.values = x.data_ptr(), out.data_ptr(), keys.data_ptr(), values.data_ptr()
         a.workspace, a.workspace_bytes = workspace.data_ptr(), 2 * workspace.numel()
         status = self._fn(ctypes.byref(a), _stream(x.device))
