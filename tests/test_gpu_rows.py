@@ -128,3 +128,15 @@ def test_layer_rows_refuses(device):
             rows.run(x, both[0], both[1], start)
     with pytest.raises(ValueError, match='overlaps'):
         rows.run(x, both[0], both[0], 0)
+
+
+def test_batches_past_the_launch_limits_are_staged(device):
+    """65536 sequences (one past a grid's z range) still run: their first rows are those of a small batch."""
+    announce('layer rows limits')
+    lay = layer('w4a16', capacity=8)
+    rows = lay._dev(device)['rows']
+    assert rows.fits(65535, 1) and rows.fits(1365, 256) and not rows.fits(65536, 1) and not rows.fits(1366, 256)
+    x = torch.randn(64, 1, 576, generator=torch.Generator().manual_seed(4)).half().to(device)
+    with torch.no_grad():
+        want = lay(x)
+        assert rel(lay(x.repeat(1024, 1, 1))[-64:], want.cpu()) <= 1e-2

@@ -449,8 +449,8 @@ bool ring_takes(const lb_linear_args *a) {
   const bool scaled = a->format != LB_FORMAT_FP16 && !(a->format == LB_FORMAT_INT8 && a->group_size == a->K);
   if (scaled && (!aligned(a->scales, 16) || ring_scale_kb(a->K / a->group_size) == 0)) return false;
   // Groups of 32, powers of two from 64 on, or one per row: a half stage of 64 codes never spans two but for 32.
-  // Byte offsets of a tile's rows are 32-bit.
-  return 64 * a->ldx * 2 <= INT32_MAX && 64 * a->K * 2 <= INT32_MAX;
+  // Byte offsets of a tile's rows, and of U, are 32-bit.
+  return 64 * a->ldx * 2 <= INT32_MAX && 64 * a->K * 2 <= INT32_MAX && (a->rank == 0 || up_ld <= INT32_MAX / 2 / a->N);
 }
 
 int ring_rt(const lb_linear_args *a, const Plan &pl) {

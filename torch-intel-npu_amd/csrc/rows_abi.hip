@@ -103,6 +103,8 @@ lb_status check_projection(const lb_layer_projection &q, int index, int64_t N, i
     return fail(LB_UNSUPPORTED, "lb_layer_rows: projection %d: ranks 8, 16, 24 or 32 with int8 weights", index);
   if (q.rank > 0 && (!q.down || !q.up || !aligned(q.down, 16) || !aligned(q.up, 16) || q.up_ld < q.rank || q.up_ld % 8 != 0))
     return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: projection %d: down / up need 16-byte alignment, up_ld >= rank a multiple of 8", index);
+  if (q.rank > 0 && q.up_ld > INT32_MAX / 2 / q.N)  // (byte offsets into U are 32-bit)
+    return fail(LB_UNSUPPORTED, "lb_layer_rows: projection %d: up_ld %lld is past 32-bit offsets", index, (long long)q.up_ld);
   return LB_OK;
 }
 

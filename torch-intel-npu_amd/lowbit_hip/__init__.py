@@ -916,7 +916,7 @@ class LayerRows:
     buffers belong to each call, so one instance may be used from several streams and threads.
     """
 
-    MAX_POSITIONS, MAX_GROUPS = 2016, 64
+    MAX_POSITIONS, MAX_GROUPS, MAX_BATCH = 2016, 64, 65535
 
     def __init__(self, projections, *, hidden, intermediate, norm1, norm2, eps, heads, kv_heads, cos, sin, scale=0.125):
         a = LayerRowsArgs()
@@ -958,6 +958,10 @@ class LayerRows:
             if pr.get('rank', 0) > MAX_RANK or (pr.get('rank', 0) and pr['format'] != 'int8'):
                 return False
         return True
+
+    def fits(self, batch, seq):
+        """Whether a call of batch x seq rows is within lb_layer_rows' launch limits."""
+        return batch <= self.MAX_BATCH and batch * seq <= (2 ** 31 - 1) // self._template.intermediate // 4
 
     def run(self, x, keys, values, start):
         """x fp16 [batch, seq, hidden] (contiguous) -> the layer's output; keys and values [batch, kv_heads,

@@ -8,8 +8,8 @@ forward / prefill / decode / reference_cpu methods and their fp16 staging (refer
 low-bit (W8 per-row, INT4/NF4 group-32, optional rank-r correction) and a layer runs as one
 lb_layer_rows call of liblowbit_hip (RMSNorm, projections, RoPE and KV append, attention, SiLU
 and residuals in seven launches, the same fp16 rounding points), for a prefill as for a decode
-step.  Layers it does not take (projections of mixed formats, capacities past 2016) run one lb_linear
-per projection with the glue as staged PyTorch-ROCm ops.
+step.  What it does not take (projections of mixed formats, capacities past 2016, more than 65535 sequences or
+349525 rows) runs one lb_linear per projection with the glue as staged PyTorch-ROCm ops.
 
 Deviations (the reference limits come from its NPU graph and are lifted):
   * rope_theta: any positive value from the config (the reference accepts only 1e5, :81);
@@ -347,7 +347,7 @@ class FrozenSmolLayer(torch.nn.Module):
         both [2, B, 3, slots, 64]."""
         state = self._dev(x.device)
         b, s, d = x.shape
-        if 'rows' in state:
+        if 'rows' in state and state['rows'].fits(b, s):
             return state['rows'].run(x.detach().contiguous(), both[0], both[1], 0)
         n1 = self._norm(x, state['norm1']).view(b * s, d)
         q = self._linear(state, n1, 'self_attn.q_proj.weight').view(b, s, HEADS, HEAD_DIM).transpose(1, 2)
@@ -394,7 +394,7 @@ class FrozenSmolLayer(torch.nn.Module):
             storage = _KVStorage(storage.both.clone(), cache.length)
         p = cache.length
         b = x.shape[0]
-        if 'rows' in state:
+        if 'rows' in state and state['rows'].fits(b, 1):
             out = state['rows'].run(x.detach().contiguous(), storage.keys, storage.values, p)
             storage.high = p + 1
             position = torch.full((1,), p + 1, dtype=torch.int32, device=x.device)
