@@ -90,3 +90,28 @@ def test_ring_strided_rows_leave_the_rest(device, columns, pitch):
     assert not np.isfinite(got[3, :columns]).all() and np.isnan(got[9, :columns]).all()
     rows = [r for r in range(m) if r not in (3, 9)]
     check(dict(p, x=p['x'][rows], m=len(rows)), got[rows][:, :columns], 'ring strided')
+
+
+# (fmt, M, N, K, group, bias): K slices of whole and ragged ends (the last stage of 32 and 96 codes, a last slice
+# shorter than the others), both row tiles, plans of tile_rows / wide_rows / the split GEMM, the lines of the rule, and
+# rows that wide_rows_kernel does not cut (11008 codes of int8)
+SLICED = [('int8', 17, 1000, 3104, 3104, True), ('int8', 32, 4096, 4096, 4096, False), ('int4', 24, 200, 4160, 64, True),
+          ('nf4', 33, 130, 3168, 3168, False), ('int4', 64, 577, 8192, 128, True), ('int8', 100, 65, 8224, 8224, False),
+          ('nf4', 129, 192, 4096, 64, True), ('int4', 20, 2048, 8192, 128, False), ('nf4', 32, 4096, 4096, 128, True),
+          ('int8', 19, 512, 11008, 11008, True), ('int4', 17, 320, 14336, 14336, False)]
+
+
+@pytest.mark.parametrize('spec', SLICED, ids=lambda s: '-'.join(map(str, s)))
+def test_ring_slices_match_oracle(device, spec):
+    """The oracle, bit-equal repeats, and rows of infinities and NaN that stay in their rows."""
+    fmt, m, n, k, group, bias = spec
+    announce('ring slices', spec)
+    p = problem(np.random.default_rng(m + n + k), fmt, m, n, k, group, rank=0, bias=bias)
+    got = run(p, device)
+    check(p, got, f'ring slices {spec}')
+    assert np.array_equal(run(p, device), got)
+    x = p['x'].copy()
+    x[1, k - 1], x[m - 1, 3] = np.inf, np.nan
+    bad = run(dict(p, x=x), device)
+    rows = [r for r in range(m) if r not in (1, m - 1)]
+    assert np.array_equal(bad[rows], got[rows]) and np.isnan(bad[m - 1]).all() and not np.isfinite(bad[1]).any()

@@ -31,8 +31,9 @@ constexpr int kRingMaxProblems = 3;
 constexpr int kRingThreads = 512;
 // RING_PLAIN: the problems' columns side by side.  RING_SILU: problems 0 and 1 are gate and up, the output is
 // fp16(fp16(silu(gate)) up).  RING_ROPE: problems 0, 1, 2 are q (rotated), k (rotated, to the cache) and v (to
-// the cache).
-enum RingMode { RING_PLAIN = 0, RING_SILU = 1, RING_ROPE = 2 };
+// the cache).  RING_SLICE: one problem, workgroup z sums codes z kslice .. of every row into fp32 partials
+// [z, M, N], which splitk_reduce_kernel adds in slice order.
+enum RingMode { RING_PLAIN = 0, RING_SILU = 1, RING_ROPE = 2, RING_SLICE = 3 };
 
 struct RingProblem {
   const uint8_t *codes;   // packed codes (fp16 weights for FMT_FP16), rows [N, K]
@@ -51,6 +52,8 @@ struct RingParams {
   const f16 *x;           // [M, ldx]
   int M, K, ldx, G, group_shift, per_row;
   int row_bytes;          // bytes of a weight row
+  int kslice;             // RING_SLICE: codes per slice, whole stages of 128
+  float *partial;         // RING_SLICE: [slices, M, N]
   RingProblem prob[kRingMaxProblems];
   // RING_ROPE: row m is position start + m % seq of sequence m / seq.
   const f16 *cos, *sin;   // [capacity, 64]
@@ -91,7 +94,8 @@ template <int BYTES> __device__ __forceinline__ int ring_swz(int r) {
 
 template <int FMT, int SCALE_KB, bool POST, bool RANKED, int RT, int MODE>
 __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
-  constexpr bool PAIR = MODE == RING_SILU, SCALED = SCALE_KB > 0;
+  constexpr bool PAIR = MODE == RING_SILU, SLICE = MODE == RING_SLICE, SCALED = SCALE_KB > 0;
+  static_assert(!(SLICE && RANKED), "a correction's z takes the whole of K");
   static_assert(!POST || SCALED, "scales to apply");
   constexpr int NP = PAIR ? 2 : 1;                     // problems a tile's weight rows come from (32 of each)
   constexpr int NV = RANKED ? NP : 0;
@@ -140,14 +144,15 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
   const RingProblem &pr = p.prob[pi];
   const int bn = ct * PART, bm = blockIdx.y * BM;
   const int rows_a = min(BM, p.M - bm);
-  const int full = p.K / 128, rest = p.K % 128, stages = full + (rest ? 1 : 0);
+  const int k0 = SLICE ? (int)blockIdx.z * p.kslice : 0, K = SLICE ? min(p.kslice, p.K - k0) : p.K;
+  const int full = K / 128, rest = K % 128, stages = full + (rest ? 1 : 0);
   auto problem = [&](int e) -> const RingProblem & { return PAIR ? p.prob[e] : pr; };
 
   // Buffer views: (base, bytes).  A wave's transfer moves a block of 1 KB: 4 rows of 256 bytes, 8 of 128 or
   // 16 of 64; lane L fills position L % (row / 16) of its row, so it reads that position's chunk of the row.
   // Block i of a wave is block wave + 4 (kg + 2 i) of the operand.
-  const f16 *xbase = p.x + (size_t)bm * p.ldx;
-  const int xbytes = ((rows_a - 1) * p.ldx + p.K) * 2;
+  const f16 *xbase = p.x + (size_t)bm * p.ldx + k0;
+  const int xbytes = ((rows_a - 1) * p.ldx + K) * 2;
   int a_off[T::A_PER];
 #pragma unroll
   for (int i = 0; i < T::A_PER; ++i) {
@@ -162,8 +167,8 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
     const int first = BLOCK_ROWS * (wave + 4 * ((T::B_SPARE ? 0 : kg) + 2 * i)), r = first + lane / CH;
     const RingProblem &q = problem(first / PART);        // a block's rows belong to one problem
     const int rows_b = min(PART, q.N - bn), n = r % PART;
-    wbase[i] = q.codes + (size_t)bn * p.row_bytes;
-    wbytes[i] = rows_b * p.row_bytes;
+    wbase[i] = q.codes + (size_t)bn * p.row_bytes + k0 * BITS / 8;
+    wbytes[i] = rows_b * p.row_bytes - k0 * BITS / 8;
     b_off[i] = n < rows_b && !(T::B_SPARE && kg == 0) ? n * p.row_bytes + 16 * ((lane % CH) ^ ring_swz<T::B_ROW>(r)) : kOutOfRange;
   }
   const int v_row = 4 * (wave + 4 * kg) + (lane >> 4);
@@ -228,7 +233,7 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
         for (int e = 0; e < 4; ++e) f.w[4 * i + e] = v[e];
       }
     }
-    if constexpr (SCALED) f.s = scales_lds[(16 * wave + j) * p.G + ((128 * t + 64 * kg + 16 * g) >> p.group_shift)];
+    if constexpr (SCALED) f.s = scales_lds[(16 * wave + j) * p.G + ((k0 + 128 * t + 64 * kg + 16 * g) >> p.group_shift)];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
 #pragma unroll
@@ -386,6 +391,18 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
     }
   }
   // D layout of the 16x16 MFMA: lane (j, g), register q -> row 4 g + q, column j.
+  if constexpr (SLICE) {
+    if (kg == 0 && wn < pr.N) {
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int m = bm + 16 * r + 4 * g + e;
+          if (m < p.M) p.partial[((size_t)blockIdx.z * p.M + m) * pr.N + wn] = acc[r][e];
+        }
+    }
+    return;
+  }
   // S2: the fp16 z of the problems, rows of 32 at a pitch of 40.  S3: the output tile, 64 columns (gate's 32, then
   // up's) in rows of 128 bytes with swizzled chunks.
   f16 *zs = reinterpret_cast<f16 *>(S2);
@@ -485,5 +502,7 @@ constexpr int ring_scale_kb(long long G) { return 128 * G <= 8 * 1024 ? 8 : 128 
 
 // Launches the kernel over `tiles` column tiles (all problems) and row tiles of 16 rt (ring_abi.hip).
 void launch_ring(const RingParams &p, int format, bool scaled, bool ranked, int rt, int tiles, hipStream_t stream);
+// The same over `slices` K slices of p.kslice codes: per-row int8, int4 / nf4 in groups of 64 and more, rt 2 or 4.
+void launch_ring_slices(const RingParams &p, int format, int rt, int tiles, int slices, hipStream_t stream);
 
 }  // namespace lb

@@ -440,6 +440,7 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 // Of the calls of up to 32 rows: 17 and more over short rows or enough columns (wide_rows / tile_rows -> ring:
 // INT8 24x14336x4096 24.4 -> 17.9, 32x8192x2048 13.0 -> 8.6, 17x1536x576 4.8 -> 4.1, INT4 32x11008x4096 20.6 -> 13.4,
 // 32x576x1536 7.5 -> 6.0, NF4 32x8192x3072 16.1 -> 10.9; but 24x1024x4096 8.8 -> 9.9, NF4 32x4096x4096 12.5 -> 14.3),
+// long rows that wide_rows_kernel does not cut (a prime number of its chunks: INT8 17x4096x11008 136 -> 25),
 // 9 to 16 over large weights (INT4 16x11008x4096 16.7 -> 11.9, NF4 12x11008x4096 20.7 -> 15.1; INT4 16x8192x3072
 // 8.7 -> 9.1), not where wide_rows_kernel adds its 4-bit K slices itself, and every call with a correction (no z
 // launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7).
@@ -460,7 +461,9 @@ int ring_rt(const lb_linear_args *a, const Plan &pl) {
   const int64_t cols = (a->N + 63) / 64;
   const int64_t t1 = (a->M + 15) / 16 * cols, t2 = (a->M + 31) / 32 * cols, t4 = (a->M + 63) / 64 * cols;
   if (pl.path != PATH_GEMM) {
-    if (a->K > 4096 || a->format == LB_FORMAT_FP16) return 0;
+    if (a->format == LB_FORMAT_FP16) return 0;
+    const bool whole = pl.path == PATH_WIDE && pl.splits == 1 && cols <= 128;
+    if (a->K > 4096 && !whole) return 0;
     const bool nf4 = a->format == LB_FORMAT_NF4, bits8 = a->format == LB_FORMAT_INT8;
     if (pl.path == PATH_WIDE && !bits8 && pl.splits <= LB_WIDE_IN_KERNEL_SLICES) return 0;
     const bool few = a->M >= 17 ? (nf4 ? cols >= 128 : a->K <= 2048 || cols >= 64)
@@ -474,6 +477,37 @@ int ring_rt(const lb_linear_args *a, const Plan &pl) {
   if (t2 <= 256 || a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
   if (t4 <= 256) return 4;
   return a->format != LB_FORMAT_NF4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES ? 4 : 0;
+}
+
+// K slices (two and more) in which ring_gemm_kernel takes a call of 17 rows and more whose plan splits K, with *rt
+// 16-row tiles a workgroup, or 0.  Their partials lie where the plan's would: never more slices than it has, in the
+// workspace the plan asks for.  One round of 256 workgroups, slices of at least four stages.
+// us, wide_rows / tile_rows / gemm4 slices or ring_gemm_kernel over the whole K -> slices, one box:
+//   INT8       24x4096x14336 23.9 -> 17.5, 32x3072x8192 15.8 -> 11.9, 24x1024x4096 8.9 -> 7.2, 40x4096x14336 31.7 -> 22.2,
+//              64x2048x8192 18.5 -> 12.0, 100x4096x14336 35.8 -> 30.7
+//   INT4 g128  24x4096x14336 19.1 -> 16.5, 32x4096x11008 26.5 -> 14.9, 64x4096x14336 31.5 -> 23.3, 100x1024x8192 18.0 -> 14.6
+//   INT4 g64   24x3072x3072 11.3 -> 8.8, 17x4096x14336 32.0 -> 16.7
+//   NF4 g128   24x4096x14336 21.0 -> 18.6, 64x4096x14336 33.9 -> 24.1, 64x1024x4096 14.0 -> 11.0
+// The lines: the second launch and the partials cost about 3 us, so rows shorter than 3072 codes (4096 from 33
+// rows on, but for NF4) stay whole (INT8 32x2048x2048 6.9 -> 7.4, 100x1024x3072 8.6 -> 9.1), as do rows of up to 4096
+// where the tiles alone give half a round (INT8 64x8192x4096 15.6 -> 18.9) or, past 32 rows, a quarter of one (INT4
+// 100x4096x4096 13.4 -> 15.6; NF4, which decodes for longer, 64x4096x4096 14.5 -> 12.4); more than 128 rows in two
+// slices (INT8 200x2048x8192 18.7 -> 20.3); and the weights of tile_rows_kernel under 16 M codes, whose slices are
+// more and add themselves (INT4 32x1024x8192 8.4 -> 9.1, 32x2048x4096 8.2 -> 9.1).
+int ring_slices(const lb_linear_args *a, const Plan &pl, int *rt) {
+  constexpr uint32_t kForce =
+      LB_FLAG_FORCE_GEMV | LB_FLAG_FORCE_GEMM | LB_FLAG_FORCE_GENERIC | LB_FLAG_FORCE_STREAM | LB_FLAG_FORCE_WIDE;
+  const bool nf4 = a->format == LB_FORMAT_NF4;
+  if ((a->flags & kForce) || pl.splits < 2 || a->M < 17 || a->rank > 0 || a->format == LB_FORMAT_FP16 || !ring_takes(a)) return 0;
+  if (a->group_size != a->K && (a->format == LB_FORMAT_INT8 || a->group_size < 64)) return 0;
+  if (a->K < (a->M <= 32 || nf4 ? 3072 : 4096) || (pl.path == PATH_TILE && a->N * a->K < (int64_t)16 << 20)) return 0;
+  *rt = a->M <= 32 ? 2 : 4;
+  const int64_t tiles = (a->M + 16 * *rt - 1) / (16 * *rt) * ((a->N + 63) / 64), stages = (a->K + 127) / 128;
+  if (a->K <= 4096 && tiles > (a->M <= 32 || nf4 ? 64 : 32)) return 0;
+  const int64_t slices = std::min<int64_t>(std::min<int64_t>(pl.splits, 256 / tiles), stages / 4);
+  if (slices < (a->M > 128 ? 3 : 2)) return 0;
+  const int64_t per = (stages + slices - 1) / slices;
+  return (int)((stages + per - 1) / per);
 }
 
 // Workspace and kernel path of the compact_groups and W8A8 variants.
@@ -851,8 +885,8 @@ void dense_fp16(int64_t M, int64_t N, int64_t K, const void *w, int64_t ldw, con
   }
 }
 
-// A PATH_GEMM call on ring_gemm_kernel (no workspace: the correction and the whole K run in the launch).
-void launch_ring_linear(const lb_linear_args *a, const LinearParams &p, int rt, hipStream_t s) {
+// A call on ring_gemm_kernel: the correction and the whole K in one launch, or K slices and their addition.
+void launch_ring_linear(const lb_linear_args *a, LinearParams p, int rt, int slices, hipStream_t s) {
   RingParams rp{};
   rp.x = p.x;
   rp.M = p.M;
@@ -878,6 +912,14 @@ void launch_ring_linear(const lb_linear_args *a, const LinearParams &p, int rt, 
   }
   const int tiles = (p.N + 63) / 64;
   for (RingProblem &r : rp.prob) r.tiles_end = tiles;
+  if (slices > 1) {
+    rp.kslice = ((p.K + 127) / 128 + slices - 1) / slices * 128;
+    rp.partial = p.partial;
+    launch_ring_slices(rp, (int)a->format, rt, tiles, slices, s);
+    p.splits = slices;
+    launch_reduce(p, s);
+    return;
+  }
   launch_ring(rp, (int)a->format, a->format != LB_FORMAT_FP16 && !p.per_row, a->rank > 0, rt, tiles, s);
 }
 
@@ -1060,8 +1102,15 @@ lb_status lb_linear(const lb_linear_args *a, void *stream) {
     launch_fused(fp, fmt, scaled, a->rank > 0, tiles, s);
     return launch_status("lb_linear");
   }
-  if (const int rt = ring_rt(a, plan)) {
-    launch_ring_linear(a, p, rt, s);
+  int rt = 0;
+  if (const int slices = ring_slices(a, plan, &rt)) {
+    p.partial = reinterpret_cast<float *>(static_cast<uint8_t *>(a->workspace) + plan.part_off);
+    launch_ring_linear(a, p, rt, slices, s);
+    return launch_status("lb_linear");
+  }
+  rt = ring_rt(a, plan);
+  if (rt > 0) {
+    launch_ring_linear(a, p, rt, 1, s);
     return launch_status("lb_linear");
   }
   if (plan.path == PATH_WIDE) {

@@ -41,4 +41,19 @@ void launch_ring(const RingParams &p, int format, bool scaled, bool ranked, int 
   }
 }
 
+template <int FMT, int SCALE_KB>
+void launch_ring_slices_t(const RingParams &p, int rt, const dim3 &grid, hipStream_t s) {
+  if (rt == 2) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 2, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
+  else hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 4, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
+}
+
+void launch_ring_slices(const RingParams &p, int format, int rt, int tiles, int slices, hipStream_t s) {
+  const dim3 grid((unsigned)tiles, (unsigned)((p.M + 16 * rt - 1) / (16 * rt)), (unsigned)slices);
+  switch (format) {
+    case FMT_INT8: launch_ring_slices_t<FMT_INT8, 0>(p, rt, grid, s); break;
+    case FMT_INT4: launch_ring_slices_t<FMT_INT4, 28>(p, rt, grid, s); break;
+    default: launch_ring_slices_t<FMT_NF4, 28>(p, rt, grid, s); break;
+  }
+}
+
 }  // namespace lb
