@@ -98,7 +98,10 @@ def test_ring_strided_rows_leave_the_rest(device, columns, pitch):
 SLICED = [('int8', 17, 1000, 3104, 3104, True), ('int8', 32, 4096, 4096, 4096, False), ('int4', 24, 200, 4160, 64, True),
           ('nf4', 33, 130, 3168, 3168, False), ('int4', 64, 577, 8192, 128, True), ('int8', 100, 65, 8224, 8224, False),
           ('nf4', 129, 192, 4096, 64, True), ('int4', 20, 2048, 8192, 128, False), ('nf4', 32, 4096, 4096, 128, True),
-          ('int8', 19, 512, 11008, 11008, True), ('int4', 17, 320, 14336, 14336, False)]
+          ('int8', 19, 512, 11008, 11008, True), ('int4', 17, 320, 14336, 14336, False),
+          # 16-row tiles: 9 to 16 rows, and 5 to 8 of NF4 and INT8
+          ('int4', 9, 3072, 8192, 128, True), ('int8', 16, 3137, 8224, 8224, False), ('nf4', 5, 4109, 11008, 64, True),
+          ('int8', 8, 3200, 14336, 14336, True)]
 
 
 @pytest.mark.parametrize('spec', SLICED, ids=lambda s: '-'.join(map(str, s)))

@@ -502,7 +502,7 @@ constexpr int ring_scale_kb(long long G) { return 128 * G <= 8 * 1024 ? 8 : 128 
 
 // Launches the kernel over `tiles` column tiles (all problems) and row tiles of 16 rt (ring_abi.hip).
 void launch_ring(const RingParams &p, int format, bool scaled, bool ranked, int rt, int tiles, hipStream_t stream);
-// The same over `slices` K slices of p.kslice codes: per-row int8, int4 / nf4 in groups of 64 and more, rt 2 or 4.
+// The same over `slices` K slices of p.kslice codes: per-row int8, int4 / nf4 in groups of 64 and more, rt 1, 2 or 4.
 void launch_ring_slices(const RingParams &p, int format, int rt, int tiles, int slices, hipStream_t stream);
 
 }  // namespace lb

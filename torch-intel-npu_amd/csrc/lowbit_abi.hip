@@ -420,6 +420,9 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 #define LB_RING_MAX_TILES 544  // ring_gemm_kernel up to this many 64 x 64 tiles (rows of at least 2048 codes)
 #endif
 
+#ifndef LB_RING_SLICE_CODES
+#define LB_RING_SLICE_CODES ((int64_t)24 << 20)  // 9..16 rows: K slices of ring_gemm_kernel from this many codes on
+#endif
 #ifndef LB_RING_MID_CODES
 #define LB_RING_MID_CODES 45000000ll  // 9..16 rows: ring_gemm_kernel from this many codes on
 #endif
@@ -479,7 +482,7 @@ int ring_rt(const lb_linear_args *a, const Plan &pl) {
   return a->format != LB_FORMAT_NF4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES ? 4 : 0;
 }
 
-// K slices (two and more) in which ring_gemm_kernel takes a call of 17 rows and more whose plan splits K, with *rt
+// K slices (two and more) in which ring_gemm_kernel takes a call whose plan splits K, with *rt
 // 16-row tiles a workgroup, or 0.  Their partials lie where the plan's would: never more slices than it has, in the
 // workspace the plan asks for.  One round of 256 workgroups, slices of at least four stages.
 // us, wide_rows / tile_rows / gemm4 slices or ring_gemm_kernel over the whole K -> slices, one box:
@@ -493,15 +496,19 @@ int ring_rt(const lb_linear_args *a, const Plan &pl) {
 // where the tiles alone give half a round (INT8 64x8192x4096 15.6 -> 18.9) or, past 32 rows, a quarter of one (INT4
 // 100x4096x4096 13.4 -> 15.6; NF4, which decodes for longer, 64x4096x4096 14.5 -> 12.4); more than 128 rows in two
 // slices (INT8 200x2048x8192 18.7 -> 20.3); and the weights of tile_rows_kernel under 16 M codes, whose slices are
-// more and add themselves (INT4 32x1024x8192 8.4 -> 9.1, 32x2048x4096 8.2 -> 9.1).
+// more and add themselves (INT4 32x1024x8192 8.4 -> 9.1, 32x2048x4096 8.2 -> 9.1).  9 to 16 rows from 24 M codes
+// (INT4 16x3072x8192 12.0 -> 10.5, 16x4096x14336 17.9 -> 15.4, NF4 21.0 -> 15.9, INT8 12x5120x13824 24.8 -> 19.5, but INT4
+// 16x4096x4096 7.4 -> 9.8, 16x2048x8192 7.8 -> 10.1), 5 to 8 rows of NF4 and INT8 from 45 M (NF4 8x4096x11008 18.9 -> 13.5,
+// 8x4096x14336 17.0 -> 16.0, INT8 17.5 -> 16.4; INT4 14.4 -> 15.4, NF4 8x3072x8192 15.6 -> 18.2).
 int ring_slices(const lb_linear_args *a, const Plan &pl, int *rt) {
   constexpr uint32_t kForce =
       LB_FLAG_FORCE_GEMV | LB_FLAG_FORCE_GEMM | LB_FLAG_FORCE_GENERIC | LB_FLAG_FORCE_STREAM | LB_FLAG_FORCE_WIDE;
   const bool nf4 = a->format == LB_FORMAT_NF4;
-  if ((a->flags & kForce) || pl.splits < 2 || a->M < 17 || a->rank > 0 || a->format == LB_FORMAT_FP16 || !ring_takes(a)) return 0;
+  if ((a->flags & kForce) || pl.splits < 2 || a->M < 5 || a->rank > 0 || a->format == LB_FORMAT_FP16 || !ring_takes(a)) return 0;
   if (a->group_size != a->K && (a->format == LB_FORMAT_INT8 || a->group_size < 64)) return 0;
   if (a->K < (a->M <= 32 || nf4 ? 3072 : 4096) || (pl.path == PATH_TILE && a->N * a->K < (int64_t)16 << 20)) return 0;
-  *rt = a->M <= 32 ? 2 : 4;
+  if (a->M <= 16 && a->N * a->K < (a->M >= 9 ? LB_RING_SLICE_CODES : a->format == LB_FORMAT_INT4 ? INT64_MAX : LB_RING_MID_CODES)) return 0;
+  *rt = a->M <= 16 ? 1 : a->M <= 32 ? 2 : 4;
   const int64_t tiles = (a->M + 16 * *rt - 1) / (16 * *rt) * ((a->N + 63) / 64), stages = (a->K + 127) / 128;
   if (a->K <= 4096 && tiles > (a->M <= 32 || nf4 ? 64 : 32)) return 0;
   const int64_t slices = std::min<int64_t>(std::min<int64_t>(pl.splits, 256 / tiles), stages / 4);

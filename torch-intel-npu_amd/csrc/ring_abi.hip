@@ -43,7 +43,8 @@ void launch_ring(const RingParams &p, int format, bool scaled, bool ranked, int 
 
 template <int FMT, int SCALE_KB>
 void launch_ring_slices_t(const RingParams &p, int rt, const dim3 &grid, hipStream_t s) {
-  if (rt == 2) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 2, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
+  if (rt == 1) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 1, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
+  else if (rt == 2) hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 2, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
   else hipLaunchKernelGGL((ring_gemm_kernel<FMT, SCALE_KB, SCALE_KB != 0, false, 4, RING_SLICE>), grid, dim3(kRingThreads), 0, s, p);
 }
 
