@@ -74,9 +74,9 @@ typedef enum lb_format {
  * gate bounds the difference to fp16(q * s)); from 5 rows, fp16(q * s).  LB_UNSUPPORTED otherwise.
  * No counterpart in the reference: the path choice is internal there. */
 #define LB_FLAG_FORCE_STREAM  0x20u
-/* The several-row GEMV on 32x32 MFMA tiles (the kernel 17..32-row calls over >= 16 MB of INT4 / NF4
- * or >= 4 MB of INT8 weights take by themselves, and 9..16-row INT4 / NF4 calls over 16..64 MB split
- * into at most 4 K slices) regardless of size: INT4/NF4/INT8 codes, no
+/* The several-row GEMV on 32x32 MFMA tiles (the kernel of 17..32-row calls over >= 16 MB of INT4 / NF4
+ * or >= 4 MB of INT8 weights, and of 9..16-row INT4 / NF4 calls over 16..64 MB split into at most 4 K
+ * slices, where the few-tile GEMM does not take them) regardless of size: INT4/NF4/INT8 codes, no
  * correction or variant, M <= 32,
  * 16-byte aligned codes and x rows, K a multiple of 512 (INT4, NF4) / 256 (INT8) up to 65536, and
  * per-row INT8 or power-of-two groups of at least 128 (INT4, NF4) / 64 (INT8) codes dividing that.
@@ -104,7 +104,8 @@ typedef enum lb_format {
  * the slices in the kernel, in the last workgroup of each block of output rows (one counter there
  * per block), instead of in a second launch, with the same result bit for bit: the 17..32-row
  * kernel (up to 4 slices, N a multiple of 4 up to 262144) and the 2..16-row one-tile kernel over
- * rows longer than it stages whole (up to 1024 workgroup columns).  lb_workspace_bytes counts the
+ * rows longer than it stages whole (up to 1024 workgroup columns).  The few-tile GEMM's slices are
+ * added in a second launch with or without the flag.  lb_workspace_bytes counts the
  * reserved bytes; a call whose plan needs no scratch needs only them.  lb_linear_noalloc ignores
  * the flag.  Calls sharing a workspace must not overlap, as for any workspace.  No counterpart in
  * the reference (its NPU graph owned its intermediates, torch_npu_lowbit.py:189-277). */

@@ -1,5 +1,5 @@
-"""GPU parity of the few-tile GEMM (ring_gemm_kernel): calls of 33 rows and more (17 where K >= N) whose grid
-is small take it without a flag, with 16, 32 or 64 rows per workgroup.
+"""GPU parity of the few-tile GEMM (ring_gemm_kernel): calls of 33 rows and more whose grid is
+small, and some of fewer rows, take it without a flag, with 16, 32 or 64 rows per workgroup, over the whole K or in slices.
 
 Bars as for every linear (rel-L2 <= 1e-3 against the oracle, the reference's rounding-budget gate); identity
 inputs with power-of-two scales are bit-exact; two calls agree bit for bit.
