@@ -226,6 +226,27 @@ def test_graph_decoder_matches_eager(device, mode):
         decoder.generate(96)
 
 
+@pytest.mark.parametrize('mode', ['stack', 'layer', 'fused', 'staged'])
+def test_graph_decoder_ignores_slots_past_the_snapshot(device, mode):
+    """Slots past a snapshot's length are another continuation's: NaN and infinities there, or left in the
+    decoder by an earlier sequence, change neither tokens nor logits."""
+    announce('graph decoder poisoned tail', mode)
+    from torch_npu_smollm import GraphDecoder
+    stack, io, _, _ = smollm_random.build(seed=5, layers=2, rank=0, theta=10000.0, capacity=48)
+    io = io.to(device)
+    with torch.no_grad():
+        _, caches = stack.prefill(io.embed_tokens(smollm_random.prompt(seed=5, length=20).to(device)))
+    decoder = GraphDecoder(stack, io, fused=mode != 'staged', layer=mode in ('layer', 'stack'),
+                           stack_kernel=mode == 'stack')
+    decoder.load(caches, 7)
+    want, logits = decoder.generate(6), decoder.logits.clone()
+    for poison in ([c.keys for c in caches] + [c.values for c in caches], decoder.keys + decoder.values):
+        for t in poison:
+            t[:, :, 20::2], t[:, :, 21::2] = float('nan'), float('inf')
+        decoder.load(caches, 7)
+        assert decoder.generate(6) == want and torch.equal(decoder.logits, logits)
+
+
 def test_config4_graph_decoder_matches_oracle(device, config4):
     """Config 4 through the graph-replayed decode step, one lb_decode_stack launch for the 30 layers
     per token: the 32 greedy tokens equal the oracle's, every step's logits are within rel-L2 1e-2

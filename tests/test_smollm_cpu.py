@@ -11,6 +11,7 @@ logits match F.rms_norm + F.linear (test_torch_npu_smollm_io.py:27-35).
 import json
 import tempfile
 from pathlib import Path
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -21,7 +22,7 @@ from oracle import smollm_oracle as so
 import smollm_random
 from torch_npu_lowbit import quantize_weight
 from torch_npu_lowbit_correction import LowRankCorrection
-from torch_npu_smollm import FrozenSmolLayer, FrozenSmolStack, _SHAPES
+from torch_npu_smollm import FrozenSmolLayer, FrozenSmolStack, GraphDecoder, _SHAPES
 from torch_npu_smollm_io import FrozenSmolIO
 
 CONFIG = dict(model_type='llama', hidden_size=576, intermediate_size=1536, num_attention_heads=9,
@@ -152,6 +153,24 @@ def test_policy_and_correction_guards(policy_weights):
     assert layer.fp16_projections == frozenset(('mlp.down_proj.weight',))
     with pytest.raises(AttributeError):
         layer.fp16_projections = ()
+
+
+@pytest.mark.parametrize('fused', [True, False])
+def test_graph_decoder_load_takes_the_valid_slots(fused):
+    """load() copies the snapshot's slots; the staged step, which multiplies every slot, finds zeros past them."""
+    decoder = GraphDecoder.__new__(GraphDecoder)
+    decoder.fused, decoder.capacity, decoder.io = fused, 8, SimpleNamespace(embedding=torch.ones(4, 576).half())
+    decoder.pos, decoder.token, decoder.h = torch.zeros(1).long(), torch.zeros(1).long(), torch.zeros(576).half()
+    decoder.keys, decoder.values = ([torch.full((1, 3, 8, 64), float('nan')).half() for _ in range(2)] for _ in range(2))
+    caches = [SimpleNamespace(length=5, keys=torch.randn(1, 3, 8, 64).half(), values=torch.randn(1, 3, 8, 64).half())
+              for _ in range(2)]
+    for c in caches:
+        c.keys[:, :, 5:], c.values[:, :, 5:] = float('nan'), float('inf')
+    decoder.load(caches, 1)
+    assert int(decoder.pos) == 5 and int(decoder.token) == 1
+    for got, c in zip(zip(decoder.keys, decoder.values), caches):
+        for dst, src in zip(got, (c.keys, c.values)):
+            assert torch.equal(dst[:, :, :5], src[:, :, :5]) and (fused or not dst[:, :, 5:].any())
 
 
 def test_checkpoint_round_trip():

@@ -869,14 +869,18 @@ class GraphDecoder:
         if not 1 <= length < self.capacity:
             raise ValueError('the snapshot leaves no free KV slot')
         targets, sources = self.keys + self.values, [c.keys for c in caches] + [c.values for c in caches]
-        if len(targets) == len(sources) and all(t.shape == s.shape for t, s in zip(targets, sources)):
+        if self.fused and len(targets) == len(sources) and all(t.shape == s.shape for t, s in zip(targets, sources)):
             # Whole buffers, contiguous: all layers' copies share launches (60 strided copies took 0.5 ms of a
-            # 16-token generation).  Slots from `length` on are written before they are read.
+            # 16-token generation).  What a later continuation wrote past `length` comes along: the fused kernels'
+            # buffers end at the position, so they read no slot before its own token has written it.
             torch._foreach_copy_(targets, sources)
         else:
             for dst_k, dst_v, cache in zip(self.keys, self.values, caches):
                 dst_k[:, :, :length].copy_(cache.keys[:, :, :length])
                 dst_v[:, :, :length].copy_(cache.values[:, :, :length])
+            if not self.fused:  # the staged attention multiplies every slot, by masked scores and zero probabilities
+                for dst in self.keys + self.values:
+                    dst[:, :, length:].zero_()
         self.pos.fill_(length)
         self.token.fill_(int(next_token))
         self.h.view(1, HIDDEN).copy_(self.io.embedding[int(next_token)].view(1, HIDDEN))
