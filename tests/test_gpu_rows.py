@@ -14,6 +14,7 @@ from conftest import announce
 from torch_npu_lowbit import QuantizedLinear, quantize_weight
 from torch_npu_lowbit_correction import LowRankCorrection
 from torch_npu_smollm import _SHAPES, FrozenSmolLayer
+from torch_npu_smollm_io import FrozenSmolIO
 
 pytestmark = pytest.mark.gpu
 
@@ -103,6 +104,29 @@ def test_rms_rows(device, rows, width):
     got = lowbit_hip.rms_rows(x.to(device), gamma.to(device)).cpu()
     # one fp16 rounding of the normalised value may fall on the other side of a tie, one of the product follows
     assert (np.abs(got.float().numpy() - want.float().numpy()) <= 2 ** -9 * np.abs(want.float().numpy()) + 2 ** -24).all()
+
+
+def test_rows_at_any_address(device):
+    """Contiguous views that begin at an odd element (2-byte aligned) give the bits of an aligned copy, through
+    forward, prefill, decode and the logits, whose norm may be such a view too."""
+    announce('rows at any address')
+    lay = layer('w8a16', 8)
+    g = torch.Generator().manual_seed(9)
+    io = FrozenSmolIO(smollm_random.config(10000.0, 1), torch.randn(49152, 576, generator=g) * 0.02,
+                      1 + 0.1 * torch.randn(576, generator=g)).to(device)
+    for batch, seq in ((1, 1), (2, 5)):
+        flat = torch.randn(batch * seq * 576 + 1, generator=g).half().to(device)
+        odd = flat[1:].view(batch, seq, 576)
+        x = odd.clone()
+        assert odd.data_ptr() % 16 and odd.is_contiguous() and x.data_ptr() % 16 == 0
+        with torch.no_grad():
+            assert torch.equal(lay(odd), lay(x)) and torch.equal(io.logits(odd), io.logits(x))
+            (a, cache), (b, _) = lay.prefill(odd), lay.prefill(x)
+            assert torch.equal(a, b)
+            assert torch.equal(lay.decode(odd[:, :1], cache)[0], lay.decode(x[:, :1].contiguous(), cache)[0])
+    want = io.logits(x)
+    io.norm = torch.cat((io.norm[:1], io.norm))[1:]
+    assert io.norm.data_ptr() % 16 and torch.equal(io.logits(x), want)
 
 
 def test_copies_of_used_modules(device):

@@ -898,9 +898,16 @@ class PreparedStack(_Prepared):
 
 
 # ---------------------------------------------------------------- several token rows
+def _aligned(t):
+    """t, contiguous and at a 16-byte address (a contiguous view may begin at any element)."""
+    t = t.detach().contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def rms_rows(x, gamma, eps=1e-5):
-    """lb_rms_rows: fp16(fp16(x * rsqrt(mean(x^2) + eps)) * gamma) of the contiguous fp16 rows of x [..., K]."""
+    """lb_rms_rows: fp16(fp16(x * rsqrt(mean(x^2) + eps)) * gamma) of the fp16 rows of x [..., K]."""
     rows, width = x.numel() // x.shape[-1], x.shape[-1]
+    x, gamma = _aligned(x), _aligned(gamma)
     _row(x, 'x', rows * width)
     _row(gamma, 'gamma', width)
     y = torch.empty_like(x)
@@ -964,8 +971,9 @@ class LayerRows:
         return batch <= self.MAX_BATCH and batch * seq <= (2 ** 31 - 1) // self._template.intermediate // 4
 
     def run(self, x, keys, values, start):
-        """x fp16 [batch, seq, hidden] (contiguous) -> the layer's output; keys and values [batch, kv_heads,
-        capacity, 64] receive slots start .. start + seq - 1."""
+        """x fp16 [batch, seq, hidden] -> the layer's output; keys and values [batch, kv_heads, capacity, 64]
+        receive slots start .. start + seq - 1."""
+        x = _aligned(x)
         a = LayerRowsArgs.from_buffer_copy(self._template)
         a.batch, a.seq, a.start, a.capacity = x.shape[0], x.shape[1], start, keys.shape[2]
         rows = x.shape[0] * x.shape[1]

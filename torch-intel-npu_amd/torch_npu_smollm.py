@@ -348,7 +348,7 @@ class FrozenSmolLayer(torch.nn.Module):
         state = self._dev(x.device)
         b, s, d = x.shape
         if 'rows' in state and state['rows'].fits(b, s):
-            return state['rows'].run(x.detach().contiguous(), both[0], both[1], 0)
+            return state['rows'].run(x, both[0], both[1], 0)
         n1 = self._norm(x, state['norm1']).view(b * s, d)
         q = self._linear(state, n1, 'self_attn.q_proj.weight').view(b, s, HEADS, HEAD_DIM).transpose(1, 2)
         k = self._linear(state, n1, 'self_attn.k_proj.weight').view(b, s, KV_HEADS, HEAD_DIM).transpose(1, 2)
@@ -395,7 +395,7 @@ class FrozenSmolLayer(torch.nn.Module):
         p = cache.length
         b = x.shape[0]
         if 'rows' in state and state['rows'].fits(b, 1):
-            out = state['rows'].run(x.detach().contiguous(), storage.keys, storage.values, p)
+            out = state['rows'].run(x, storage.keys, storage.values, p)
             storage.high = p + 1
             position = torch.full((1,), p + 1, dtype=torch.int32, device=x.device)
             return out, SmolKVCache(self._cache_owner, cache._sequence, storage.keys, storage.values, p + 1, position, storage)

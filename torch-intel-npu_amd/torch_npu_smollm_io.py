@@ -91,7 +91,7 @@ class FrozenSmolIO(torch.nn.Module):
             raise ValueError('Output head requires nonempty FP16 (B,S,576) hidden states')
         self._check(hidden.device)
         normalized = (self.normalize(hidden) if hidden.device.type == 'cpu'
-                      else lowbit_hip.rms_rows(hidden.detach().contiguous(), self.norm))
+                      else lowbit_hip.rms_rows(hidden, self.norm))
         b, s, _ = hidden.shape
         if self.head is not None:
             return self._quantized_logits(normalized.reshape(b * s, 576)).view(b, s, self.vocab_size)
