@@ -268,7 +268,7 @@ lb_status lb_rms_rows(const void *x, const void *gamma, void *y, int64_t M, int6
  * is start = 0, a decode step seq = 1.  Seven launches (five for one row in all) with the staging of lb_decode_layer
  * (torch_npu_smollm.py:142-193); the counterpart of the reference's prefill and decode graphs of a
  * layer (:195-340, :506-544) for any batch and length.  Limits: hidden = 64 heads <= 4096,
- * intermediate a multiple of 32, at most 2016 positions; q, k, v share a format and group, gate and up
+ * intermediate a multiple of 32, start + seq at most 2016 (capacity may be larger); q, k, v share a format and group, gate and up
  * share one; int8 per row with ranks 0, 8, .., 32, or int4 / nf4 with power-of-two groups >= 32 (at most
  * 64 per row) or fp16, without corrections (LB_UNSUPPORTED otherwise).
  */

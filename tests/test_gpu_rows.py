@@ -13,7 +13,7 @@ import smollm_random
 from conftest import announce
 from torch_npu_lowbit import QuantizedLinear, quantize_weight
 from torch_npu_lowbit_correction import LowRankCorrection
-from torch_npu_smollm import _SHAPES, FrozenSmolLayer
+from torch_npu_smollm import _ROWS_ORDER, _SHAPES, FrozenSmolLayer
 from torch_npu_smollm_io import FrozenSmolIO
 
 pytestmark = pytest.mark.gpu
@@ -152,6 +152,23 @@ def test_layer_rows_refuses(device):
             rows.run(x, both[0], both[1], start)
     with pytest.raises(ValueError, match='overlaps'):
         rows.run(x, both[0], both[0], 0)
+
+
+def test_one_row_over_a_long_cache(device):
+    """A cache of 60000 slots, whose scores would not fit in LDS: one row at slot 10 gives the bits of a short cache."""
+    announce('one row, long cache')
+    outs = []
+    for capacity in (16, 60000):
+        lay = layer('w8a16', 8, capacity=capacity)
+        state = lay._dev(device)
+        rows = lowbit_hip.LayerRows([state['lin'][n] for n in _ROWS_ORDER], hidden=576, intermediate=1536,
+                                    norm1=state['norm1'], norm2=state['norm2'], eps=1e-5, heads=9, kv_heads=3,
+                                    cos=state['cos'], sin=state['sin'])
+        x = torch.randn(1, 11, 576, generator=torch.Generator().manual_seed(6)).half().to(device)
+        keys, values = torch.zeros(2, 1, 3, capacity, 64, dtype=torch.float16, device=device)
+        rows.run(x[:, :10], keys, values, 0)
+        outs.append((rows.run(x[:, 10:], keys, values, 10), keys[:, :, :16].clone(), values[:, :, :16].clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
 
 
 def test_batches_past_the_launch_limits_are_staged(device):

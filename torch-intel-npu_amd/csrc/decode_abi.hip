@@ -673,8 +673,8 @@ void launch_stream(const StreamParams &p, int format, bool scaled, int ns, hipSt
 }
 
 void launch_decode_attention(const AttnParams &p, hipStream_t s) {
-  hipLaunchKernelGGL(decode_attention_kernel, dim3((unsigned)p.heads, kAttnDimSlices), dim3(256),
-                     (size_t)p.capacity * sizeof(float), s, p);
+  const size_t scores = p.position ? (size_t)p.capacity : (size_t)p.slot + 1;  // the kernel keeps scores 0 .. position
+  hipLaunchKernelGGL(decode_attention_kernel, dim3((unsigned)p.heads, kAttnDimSlices), dim3(256), scores * sizeof(float), s, p);
 }
 
 void launch_fused(const FusedParams &p, int format, bool scaled, bool ranked, int tiles, hipStream_t s) {
