@@ -229,6 +229,46 @@ def test_decode_attention_argument_errors(over, needle, status):
     assert needle in lib.lb_last_error().decode()
 
 
+def layer_rows(**over):
+    """A valid lb_layer_rows call: one row of a SmolLM W8 layer at slot 10 of a cache of 64."""
+    a = lowbit_hip.LayerRowsArgs()
+    a.struct_size = ctypes.sizeof(a)
+    a.batch, a.seq, a.start, a.capacity = 1, 1, 10, 64
+    a.hidden, a.intermediate, a.heads, a.kv_heads, a.eps, a.scale = 576, 1536, 9, 3, 1e-5, 0.125
+    a.x, a.out, a.norm1, a.norm2, a.cos, a.sin = 0x10000, 0x11000, 0x12000, 0x13000, 0x20000, 0x30000
+    a.keys, a.values, a.workspace, a.workspace_bytes = 0x100000, 0x200000, 0x300000, 1 << 20
+    for i, (n, k) in enumerate(((576, 576), (192, 576), (192, 576), (576, 576), (1536, 576), (1536, 576), (576, 1536))):
+        q = a.proj[i]
+        q.format, q.group_size, q.N, q.K = lowbit_hip.FORMATS['int8'], k, n, k
+        q.codes, q.scales = 0x1000000 * (i + 1), 0x1000000 * (i + 1) + 0x800000
+        q.rank, q.down, q.up, q.up_ld = 8, 0x1000000 * (i + 1) + 0x900000, 0x1000000 * (i + 1) + 0xa00000, 8
+    for key, value in over.items():
+        setattr(a, key, value)
+    return a
+
+
+@pytest.mark.parametrize('over,needle,status', [
+    (dict(struct_size=8), 'struct_size', lowbit_hip.INVALID_ARGUMENT),
+    (dict(batch=65536), 'batch', lowbit_hip.INVALID_ARGUMENT),
+    (dict(start=64), 'capacity', lowbit_hip.INVALID_ARGUMENT),
+    (dict(start=2 ** 63 - 1), 'capacity', lowbit_hip.INVALID_ARGUMENT),   # start + seq past 64 bits
+    (dict(seq=2 ** 62, batch=4), 'capacity', lowbit_hip.INVALID_ARGUMENT),
+    (dict(capacity=2 ** 31), 'capacity', lowbit_hip.INVALID_ARGUMENT),    # past the kernels' 32 bits
+    (dict(start=2016, capacity=4096), 'positions', lowbit_hip.UNSUPPORTED),
+    (dict(heads=9 + 3 * 2 ** 58), 'heads', lowbit_hip.INVALID_ARGUMENT),      # 64 heads past 64 bits
+    (dict(kv_heads=2), 'kv_heads', lowbit_hip.INVALID_ARGUMENT),
+    (dict(intermediate=1540), 'intermediate', lowbit_hip.INVALID_ARGUMENT),
+    (dict(x=0x10008), 'x must', lowbit_hip.INVALID_ARGUMENT),
+    (dict(workspace_bytes=100), 'workspace', lowbit_hip.INVALID_ARGUMENT),
+    (dict(out=0x10000), 'out overlaps x', lowbit_hip.INVALID_ARGUMENT),
+    (dict(values=0x100000), 'keys overlaps values', lowbit_hip.INVALID_ARGUMENT),
+])
+def test_layer_rows_argument_errors(over, needle, status):
+    lib = lowbit_hip.library()
+    assert lib.lb_layer_rows(ctypes.byref(layer_rows(**over)), None) == status, lib.lb_last_error().decode()
+    assert needle in lib.lb_last_error().decode()
+
+
 def test_argmax_next_argument_errors():
     lib = lowbit_hip.library()
     ok = (0x10000, 1000, 0x100000, 64, 0x20000, 0x30000, 0x31000, 0x32000, 8)

@@ -210,14 +210,15 @@ lb_status lb_layer_rows(const lb_layer_rows_args *a, void *stream) {
   if (!a) return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: args is NULL");
   if (a->struct_size < sizeof(lb_layer_rows_args))
     return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: struct_size %u < %zu", a->struct_size, sizeof(lb_layer_rows_args));
-  const int64_t H = a->hidden, I = a->intermediate, M = a->batch * a->seq, kv = 64 * a->kv_heads;
-  if (a->batch < 1 || a->seq < 1 || a->start < 0 || a->batch > 65535 || a->capacity < 1 ||
-      a->start + a->seq > a->capacity)
-    return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: batch, seq >= 1 and start + seq <= capacity required");
-  if (a->heads < 1 || a->kv_heads < 1 || a->heads % a->kv_heads != 0 || H != 64 * a->heads || H > kRowsMaxHidden || I < 32 ||
-      I % 32 != 0 || I > 65536)
+  // Comparisons that no 64-bit argument overflows; the products and sums below are of checked values.
+  if (a->batch < 1 || a->batch > 65535 || a->seq < 1 || a->start < 0 || a->capacity < a->seq || a->capacity > INT32_MAX ||
+      a->start > a->capacity - a->seq)
+    return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: batch 1..65535, seq >= 1 and start + seq <= capacity <= 2^31 - 1 required");
+  if (a->hidden < 64 || a->hidden > kRowsMaxHidden || a->heads < 1 || a->heads > kRowsMaxHidden / 64 || a->hidden != 64 * a->heads ||
+      a->kv_heads < 1 || a->heads % a->kv_heads != 0 || a->intermediate < 32 || a->intermediate % 32 != 0 || a->intermediate > 65536)
     return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: hidden = 64 heads <= %d, heads a multiple of kv_heads, intermediate a "
-                "multiple of 32", kRowsMaxHidden);
+                "multiple of 32 up to 65536", kRowsMaxHidden);
+  const int64_t H = a->hidden, I = a->intermediate, M = a->batch * a->seq, kv = 64 * a->kv_heads;
   if (a->start + a->seq > kAttendMaxKeys || M > INT32_MAX / I / 4)
     return fail(LB_UNSUPPORTED, "lb_layer_rows: at most %d positions", kAttendMaxKeys);
   const struct { const void *p; const char *name; } pointers[] = {
