@@ -262,6 +262,10 @@ def layer_rows(**over):
     (dict(workspace_bytes=100), 'workspace', lowbit_hip.INVALID_ARGUMENT),
     (dict(out=0x10000), 'out overlaps x', lowbit_hip.INVALID_ARGUMENT),
     (dict(values=0x100000), 'keys overlaps values', lowbit_hip.INVALID_ARGUMENT),
+    (dict(out=0x1000000 + 576 * 576 - 16), 'out overlaps codes of projection 0', lowbit_hip.INVALID_ARGUMENT),
+    (dict(keys=0x7800000), 'keys overlaps scales of projection 6', lowbit_hip.INVALID_ARGUMENT),
+    (dict(values=0x2900000 + 8 * 576 * 2 - 16), 'values overlaps down of projection 1', lowbit_hip.INVALID_ARGUMENT),
+    (dict(workspace=0x6a00000), 'workspace overlaps up of projection 5', lowbit_hip.INVALID_ARGUMENT),
 ])
 def test_layer_rows_argument_errors(over, needle, status):
     lib = lowbit_hip.library()

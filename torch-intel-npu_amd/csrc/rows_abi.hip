@@ -246,6 +246,19 @@ lb_status lb_layer_rows(const lb_layer_rows_args *a, void *stream) {
     for (int k = i + 1; k < 4; ++k)
       if (overlaps(outs[i], outs[k])) return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: %s overlaps %s", outs[i].name, outs[k].name);
   }
+  for (int i = 0; i < 7; ++i) {
+    const lb_layer_projection &q = a->proj[i];
+    const bool dense = q.format == LB_FORMAT_FP16;
+    const size_t codes = (size_t)q.N * q.K, ranked = q.rank > 0;
+    const Range weights[] = {
+        range_of(q.codes, dense ? 2 * codes : q.format == LB_FORMAT_INT8 ? codes : codes / 2, "codes"),
+        range_of(q.scales, dense ? 0 : codes / q.group_size * 2, "scales"), range_of(q.down, (size_t)(q.rank * q.K * 2), "down"),
+        range_of(q.up, ranked * (size_t)((q.N - 1) * q.up_ld + q.rank) * 2, "up")};
+    for (const Range &out : outs)
+      for (const Range &r : weights)
+        if (overlaps(out, r))
+          return fail(LB_INVALID_ARGUMENT, "lb_layer_rows: %s overlaps %s of projection %d", out.name, r.name, i);
+  }
 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (one_row(a)) {
