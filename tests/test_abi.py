@@ -648,3 +648,34 @@ print('ok')
                          capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.strip().endswith('ok'), out.stdout + out.stderr
     assert not lowbit_hip.failed()   # this process is untouched
+
+
+@pytest.mark.parametrize('bound', [False, True])
+def test_call_workspace_keeps_the_zeroed_promise(monkeypatch, bound):
+    """linear() and BoundLinear with FLAG_ZEROED_WORKSPACE allocate a cleared workspace (its counters would start
+    anywhere otherwise); the launch is replaced by a look at what it would have been given."""
+    seen = []
+
+    class Recorder:
+        lb_workspace_bytes = lowbit_hip.library().lb_workspace_bytes
+
+        @staticmethod
+        def lb_linear(ref, stream):
+            a = ref._obj
+            seen.append((a.flags, ctypes.string_at(a.workspace, lowbit_hip.ZEROED_WORKSPACE_BYTES)))
+            return lowbit_hip.OK
+
+    dirty = torch.empty
+    monkeypatch.setattr(lowbit_hip, 'library', Recorder)
+    monkeypatch.setattr(lowbit_hip, '_stream', lambda device: None)
+    monkeypatch.setattr(lowbit_hip, 'check_operands', lambda *a, **k: None)
+    monkeypatch.setattr(torch, 'empty', lambda *a, **k: dirty(*a, **k).fill_(85))
+    m, n, k = 16, 1024, 14336   # K slices of the tiled rows
+    x, codes, scales = torch.zeros(m, k).half(), torch.zeros(n * k // 2, dtype=torch.uint8), torch.ones(n, k // 128).half()
+    spec = dict(format='int4', N=n, K=k, group_size=128, flags=lowbit_hip.FLAG_ZEROED_WORKSPACE)
+    if bound:
+        lowbit_hip.BoundLinear(codes, scales, **spec)(x)
+    else:
+        lowbit_hip.linear(x, codes, scales, **spec)
+    (flags, head), = seen
+    assert flags & lowbit_hip.FLAG_ZEROED_WORKSPACE and not any(head)

@@ -384,6 +384,13 @@ def workspace_bytes(args):
     return size.value
 
 
+def _call_workspace(need, flags, device):
+    """The workspace of one call.  Not zeroed unless the caller's flags promise it: clearing it would be a launch,
+    as the addition of K slices that it saves is."""
+    allocate = torch.zeros if flags & FLAG_ZEROED_WORKSPACE else torch.empty
+    return allocate(need, dtype=torch.uint8, device=device)
+
+
 def linear(x, codes, scales, *, format, N, K, group_size, bias=None, down=None, up=None, rank=0, flags=0,
            out=None, workspace=None, activation_scale=None):
     """y[M,N] fp16 = x . dequant(W)^T (+bias) (+fp16(fp16(x.V^T).U^T)) on the current stream.
@@ -408,8 +415,7 @@ def linear(x, codes, scales, *, format, N, K, group_size, bias=None, down=None, 
     need = workspace_bytes(args)
     if need:
         if workspace is None or workspace.numel() < need:
-            # Not a zeroed one: clearing it would be a launch, as the addition of K slices it saves is.
-            workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
+            workspace = _call_workspace(need, args.flags, x.device)
         args.workspace, args.workspace_bytes = _ptr(workspace), workspace.numel()
     _check(library().lb_linear(ctypes.byref(args), _stream(x.device)), 'lb_linear')
     return y
@@ -452,7 +458,7 @@ class BoundLinear:
                 self._needs.clear()
             self._needs[key] = need
         if need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=self._device)
+            workspace = _call_workspace(need, args.flags, self._device)
             args.workspace, args.workspace_bytes = workspace.data_ptr(), need
         status = self._fn(ctypes.byref(args), _stream(self._device))
         if status != OK:
