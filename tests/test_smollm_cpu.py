@@ -9,6 +9,7 @@ projections use the original fp16 weight (test_torch_npu_smollm_policy.py:65-74)
 logits match F.rms_norm + F.linear (test_torch_npu_smollm_io.py:27-35).
 """
 import json
+import pickle
 import tempfile
 from pathlib import Path
 from types import SimpleNamespace
@@ -20,9 +21,9 @@ import torch.nn.functional as F
 
 from oracle import smollm_oracle as so
 import smollm_random
-from torch_npu_lowbit import quantize_weight
+from torch_npu_lowbit import QuantizedLinear, quantize_weight
 from torch_npu_lowbit_correction import LowRankCorrection
-from torch_npu_smollm import FrozenSmolLayer, FrozenSmolStack, GraphDecoder, _SHAPES
+from torch_npu_smollm import FrozenSmolLayer, FrozenSmolStack, GraphDecoder, _KVStorage, _SHAPES
 from torch_npu_smollm_io import FrozenSmolIO
 
 CONFIG = dict(model_type='llama', hidden_size=576, intermediate_size=1536, num_attention_heads=9,
@@ -171,6 +172,21 @@ def test_graph_decoder_load_takes_the_valid_slots(fused):
     for got, c in zip(zip(decoder.keys, decoder.values), caches):
         for dst, src in zip(got, (c.keys, c.values)):
             assert torch.equal(dst[:, :, :5], src[:, :, :5]) and (fused or not dst[:, :, 5:].any())
+
+
+def test_modules_and_caches_pickled_before_load():
+    """State of the first releases: a module without bound calls, a cache storage of two tensors.  Current ones go
+    round too, and keep keys and values halves of one tensor."""
+    module = QuantizedLinear(quantize_weight(torch.randn(4, 32), format='int4', group_size=32))
+    old = QuantizedLinear.__new__(QuantizedLinear)
+    old.__setstate__({k: v for k, v in module.__dict__.items() if k != '_bound'})
+    assert old._bound == {} and pickle.loads(pickle.dumps(module))._bound == {}
+    keys, values = torch.randn(2, 1, 3, 8, 64).half()
+    storage = _KVStorage.__new__(_KVStorage)
+    storage.__setstate__(dict(keys=keys, values=values, high=5))
+    for s in (storage, pickle.loads(pickle.dumps(storage))):
+        assert s.high == 5 and torch.equal(s.keys, keys) and torch.equal(s.values, values)
+        assert s.keys.data_ptr() == s.both.data_ptr() and s.values.data_ptr() == s.both[1].data_ptr()
 
 
 def test_checkpoint_round_trip():

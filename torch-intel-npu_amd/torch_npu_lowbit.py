@@ -275,6 +275,10 @@ class QuantizedLinear(torch.nn.Module):
         """Copies and pickles bind their own device calls (those hold raw pointers)."""
         return {**self.__dict__, '_bound': {}}
 
+    def __setstate__(self, state):
+        """Also of modules pickled before they bound their calls."""
+        super().__setstate__({**state, '_bound': {}})
+
     def _device_bias(self, device):
         if self._bias is None:
             return None

@@ -87,6 +87,10 @@ class _KVStorage:
         self.both, self.high = both, high
         self.keys, self.values = both[0], both[1]
 
+    def __setstate__(self, state):
+        """Also of storage pickled as two tensors."""
+        self.__init__(state['both'] if 'both' in state else torch.stack((state['keys'], state['values'])), state['high'])
+
 
 @dataclass(frozen=True, eq=False)
 class SmolKVCache:
