@@ -31,6 +31,13 @@ CASES = [
     ('int4', 20, 4160, 2560, 32, 0, True), ('nf4', 20, 8190, 256, 128, 0, False), ('int4', 9, 11072, 4096, 128, 0, False),
     ('int8', 2, 100, 96, 96, 8, True), ('int8', 16, 577, 640, 640, 32, False), ('int8', 19, 64, 4096, 4096, 16, False),
     ('int4', 5, 130, 320, 64, 24, True), ('nf4', 32, 70, 96, 32, 32, False),
+    # past one round of 64-row tiles, where the kernel is estimated the faster one and where not; 17 rows over two rounds
+    ('int4', 1000, 2000, 2048, 64, 0, True), ('int8', 50, 16500, 2080, 2080, 0, False), ('int8', 320, 4900, 2048, 2048, 0, True),
+    ('int4', 320, 6912, 2048, 64, 0, False), ('int8', 17, 17000, 2048, 2048, 0, True),
+    # both sides of the lines of short rows, of pairs of tiles, of groups of 32 and of 9 to 16 rows
+    ('int4', 340, 2740, 512, 64, 0, False), ('int4', 340, 2740, 544, 32, 0, True), ('nf4', 321, 2750, 384, 64, 0, True),
+    ('int4', 19, 7588, 640, 128, 0, False), ('int4', 19, 7000, 704, 64, 0, True), ('nf4', 70, 90, 3072, 32, 0, True),
+    ('nf4', 20, 8300, 640, 64, 0, False), ('nf4', 20, 8300, 672, 32, 0, True), ('int8', 9, 17000, 2816, 2816, 0, False),
 ]
 
 
@@ -48,7 +55,7 @@ def test_ring_fp16_rows(device):
     """fp16 weights (no scales) against a double product, a ragged last stage included."""
     announce('ring fp16')
     rng = np.random.default_rng(3)
-    for m, n, k in ((40, 70, 96), (256, 576, 576), (65, 300, 1536)):
+    for m, n, k in ((40, 70, 96), (256, 576, 576), (65, 300, 1536), (100, 2050, 4128), (330, 2700, 3104), (330, 2700, 544)):
         x = rng.standard_normal((m, k)).astype(np.float16)
         w = (rng.standard_normal((n, k)) * 0.02).astype(np.float16)
         y = lowbit_hip.linear(to_dev(x, device), to_dev(w, device), None, format='fp16', N=n, K=k, group_size=k)

@@ -417,7 +417,7 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 }
 
 #ifndef LB_RING_MAX_TILES
-#define LB_RING_MAX_TILES 544  // ring_gemm_kernel up to this many 64 x 64 tiles (rows of at least 2048 codes)
+#define LB_RING_MAX_TILES 544  // ring_gemm_kernel past one round of 64-row tiles (32-row with a correction): at most this
 #endif
 
 #ifndef LB_RING_SLICE_CODES
@@ -436,17 +436,28 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 //              256x4096x4096 25.9 -> 18.8, 48x14336x4096 33.8 -> 18.9
 //   NF4 g64    500x960x2560 15.6 -> 11.8, 333x2560x960 10.5 -> 8.4, 64x8192x3072 19.8 -> 13.6
 //   INT8       700x576x1536 11.8 -> 7.2, 256x576x576 with rank 32 21.2 -> 6.1, 100x2569x3136 rank 8 54.0 -> 12.4
-// Past one round: up to two of INT4 / INT8 / fp16 rows of 2048 codes or more (512x4096x4096 37.2 -> 34.2,
-// 1024x2048x2048 27.6 -> 21.0, 600x2048x2048 20.2 -> 19.2; shorter rows 500x2560x960 11.3 -> 12.5, NF4, whose
-// table reads load LDS, 512x4096x4096 38.7 -> 42.2).  Long rows stay on split K where few workgroups would walk
-// them (INT4 40x2048x8192 18.5 -> 20.0) and, for NF4, past 4096 codes (300x2048x8192 32.3 -> 38.6).
+// Past one round the second one costs as much as the first, however few its tiles: ring_past_one_round weighs both
+// kernels.  Long rows stay on split K where few workgroups would walk them (INT4 40x2048x8192 18.5 -> 20.0, 64-row
+// tiles in groups 266x2048x8192 31.4 -> 35.3; NF4 in groups of 32 already from 3072 codes on, 462x76x4096 12.6 -> 18.2)
+// and, for NF4, whose table reads load LDS, past 4096 codes (300x2048x8192 32.3 -> 38.6).  So does fp16, whose weights
+// gemm4_kernel's larger tiles read fewer times, past 3072 codes in 64-row tiles (513x1424x12096 43.1 -> 68.6; but
+// 801x769x2176 18.6 -> 16.8, one row of tiles 62x14336x4096 32.3 -> 25.6) and past 4096 in 32-row ones over many columns
+// whose tiles of one column meet on different XCDs (55x6574x9152 29.8 -> 37.0; 178x2048x8192 22.4 -> 19.4,
+// 480x657x5952 23.3 -> 19.6).  Full rounds of 64-row tiles need rows that outlast filling the ring (INT4 186x4546x512
+// 6.9 -> 7.7, 212x2944x704 9.4 -> 7.0; INT8 and NF4 682x1166x256 6.2 -> 7.0, 562x946x448 7.2 -> 6.9; in groups of 32,
+// which gemm4_kernel scales code by code, 310x3089x256 6.1 -> 7.3, 474x1439x288 7.4 -> 7.0).
 // Of the calls of up to 32 rows: 17 and more over short rows or enough columns (wide_rows / tile_rows -> ring:
 // INT8 24x14336x4096 24.4 -> 17.9, 32x8192x2048 13.0 -> 8.6, 17x1536x576 4.8 -> 4.1, INT4 32x11008x4096 20.6 -> 13.4,
 // 32x576x1536 7.5 -> 6.0, NF4 32x8192x3072 16.1 -> 10.9; but 24x1024x4096 8.8 -> 9.9, NF4 32x4096x4096 12.5 -> 14.3),
-// long rows that wide_rows_kernel does not cut (a prime number of its chunks: INT8 17x4096x11008 136 -> 25),
-// 9 to 16 over large weights (INT4 16x11008x4096 16.7 -> 11.9, NF4 12x11008x4096 20.7 -> 15.1; INT4 16x8192x3072
-// 8.7 -> 9.1), not where wide_rows_kernel adds its 4-bit K slices itself, and every call with a correction (no z
-// launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7).
+// long rows that wide_rows_kernel does not cut (a prime number of its chunks: INT8 17x4096x11008 136 -> 25), 9 to 16
+// over large weights in one round (INT4 16x11008x4096 16.7 -> 11.9, NF4 12x11008x4096 20.7 -> 15.1; INT4
+// 16x8192x3072 8.7 -> 9.1) or where a second one is over half full and tile_rows_kernel does not take them (9x19834x3712
+// 22.3 -> 31.2, 11x28779x3712 35.6 -> 31.1; INT8 11x25759x2048 16.6 -> 20.4), and every call
+// with a correction (no z launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7).
+// Not where wide_rows_kernel cuts 4-bit rows into few slices, nor where 17 rows and more suit tile_rows_kernel: one
+// round of its pairs of tiles (INT4 19x7588x640 4.6 -> 6.0, 17x7939x960 4.9 -> 6.8; 23x5898x704 9.6 -> 5.5 before the
+// pairs fill it), and the lengths it stages exactly, 1024 over few columns (INT4 23x1878 5.3 -> 5.8, but 28x1984x896
+// 5.6 -> 5.0) and, for NF4, up to 640 (23x13694 6.2 -> 6.7, but 17x8487x768 9.0 -> 7.0).
 bool ring_takes(const lb_linear_args *a) {
   const int64_t up_ld = a->up_ld == 0 ? a->rank : a->up_ld;
   if (a->rank > 0 && (a->rank > 32 || a->rank % 8 != 0 || !aligned(a->down, 16) || !aligned(a->up, 16) || up_ld % 8 != 0)) return false;
@@ -457,29 +468,64 @@ bool ring_takes(const lb_linear_args *a) {
   return 64 * a->ldx * 2 <= INT32_MAX && 64 * a->K * 2 <= INT32_MAX && (a->rank == 0 || up_ld <= INT32_MAX / 2 / a->N);
 }
 
+// Whether ring_gemm_kernel takes a grid of `tiles` 64-row tiles, more than one round of 256 workgroups, by an estimate
+// of both kernels' us.  Its own: rounds x K at 3.4 a thousand codes (INT8 in groups 3.6; per row, without scales in the
+// loop, 3.0), and 7.5 to start, fill and drain.  gemm4_kernel's: rounds x slice length at 7.7 a thousand codes for
+// 128 x 128 tiles, up to 2.9 more as the last round fills, 3.7 for 64 x 64 ones, and its slices' partials at 2.3 a
+// million values beside a launch.  Fitted to 1459 shapes of 33 to 2048 rows, K 2048 to 14336 and 257 to 544 tiles, both
+// sides of each measured: the estimates deviate by 5 to 6%, the choice leaves about 20 of them more than 3% slower than
+// gemm4_kernel (taking all of them 540, by up to 1.5 times) and saves 7% over all.  INT4 g64 320x6912x4096 stays at 41.5
+// (ring 53.0), 512x4096x14336 at 92.7 (102.3), 1024x2048x2048 goes 24.9 -> 21.5, 64x32832x4096 66.0 -> 54.9.  NF4 and
+// fp16 measured slower throughout (512x4096x4096 38.7 -> 42.2, 748x1536x2752 22.1 -> 31.2), rows under 2048 codes too
+// (INT4 500x2560x960 11.3 -> 12.5).
+bool ring_past_one_round(const lb_linear_args *a, int64_t tiles) {
+  if (a->format == LB_FORMAT_NF4 || a->format == LB_FORMAT_FP16 || a->K < 2048 || tiles > LB_RING_MAX_TILES) return false;
+  const auto rounds = [](int64_t wgs) { return (double)((wgs + 255) / 256); };
+  const GemmShape gs = gemm_shape(a->M, a->N, a->K, 1, true);
+  const bool small = gs.kind == GEMM_64 || gs.kind == GEMM_64_K32;
+  const int64_t edge = small ? 64 : 128, wgs = (a->M + edge - 1) / edge * ((a->N + edge - 1) / edge) * gs.splits;
+  const double codes = 1e-3 * gs.kslice, fill = wgs / 256.0 - (rounds(wgs) - 1);
+  const double gemm4 = 4.0 + codes * (small ? 3.7 * rounds(wgs) : 7.7 * rounds(wgs) + 2.9 * fill) +
+                       (gs.splits > 1 ? 1.0 + 2.3e-6 * a->M * a->N * gs.splits : 0.0);
+  const bool bits8 = a->format == LB_FORMAT_INT8, per_row = bits8 && a->group_size == a->K;
+  return 7.5 + (per_row ? 3.0 : bits8 ? 3.6 : 3.4) * 1e-3 * a->K * rounds(tiles) < gemm4;
+}
+
 int ring_rt(const lb_linear_args *a, const Plan &pl) {
   constexpr uint32_t kForce =
       LB_FLAG_FORCE_GEMV | LB_FLAG_FORCE_GEMM | LB_FLAG_FORCE_GENERIC | LB_FLAG_FORCE_STREAM | LB_FLAG_FORCE_WIDE;
   if ((a->flags & kForce) || pl.path == PATH_GENERIC || pl.path == PATH_ROW || pl.path == PATH_STREAM || !ring_takes(a)) return 0;
   const int64_t cols = (a->N + 63) / 64;
   const int64_t t1 = (a->M + 15) / 16 * cols, t2 = (a->M + 31) / 32 * cols, t4 = (a->M + 63) / 64 * cols;
+  const bool nf4 = a->format == LB_FORMAT_NF4, dense = a->format == LB_FORMAT_FP16, bits8 = a->format == LB_FORMAT_INT8;
+  const bool groups32 = !dense && a->group_size == 32;
   if (pl.path != PATH_GEMM) {
-    if (a->format == LB_FORMAT_FP16) return 0;
+    if (dense) return 0;
     const bool whole = pl.path == PATH_WIDE && pl.splits == 1 && cols <= 128;
     if (a->K > 4096 && !whole) return 0;
-    const bool nf4 = a->format == LB_FORMAT_NF4, bits8 = a->format == LB_FORMAT_INT8;
     if (pl.path == PATH_WIDE && !bits8 && pl.splits <= LB_WIDE_IN_KERNEL_SLICES) return 0;
-    const bool few = a->M >= 17 ? (nf4 ? cols >= 128 : a->K <= 2048 || cols >= 64)
-                                : a->M >= 9 && a->N * a->K >= LB_RING_MID_CODES;
+    const bool pairs = (a->N + 15) / 16 >= 2 * LB_TILE_ROWS_MIN_WGS && cols <= 128;  // (tile_rows_per_wg)
+    const bool staged = nf4 ? a->K <= 640 : a->K > 992 && cols <= 64;
+    const bool tiled = pl.path == PATH_TILE && pl.splits == 1 && (pairs || staged);
+    const bool few = a->M >= 17 ? !tiled && (nf4 ? cols >= 128 : a->K <= 2048 || cols >= 64)
+                                : a->M >= 9 && a->N * a->K >= LB_RING_MID_CODES &&
+                                      (cols <= 256 || (cols > 384 && cols <= 512 && pl.path != PATH_TILE));
     if (!few && a->rank == 0) return 0;
   } else {
-    if (a->format == LB_FORMAT_NF4 && a->K > 4096) return 0;
+    if (nf4 && a->K > 4096) return 0;
     if (a->K > 4096 && t1 <= 128) return 0;
+    if (nf4 && groups32 && a->K >= 3072 && a->K % 64 == 0 && t1 <= 128 && a->rank == 0) return 0;
   }
   if (t1 <= 256) return 1;
-  if (t2 <= 256 || a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
-  if (t4 <= 256) return 4;
-  return a->format != LB_FORMAT_NF4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES ? 4 : 0;
+  if (a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
+  if (t2 <= 256) return dense && a->K > 4096 && cols > 24 && cols % 8 != 0 ? 0 : 2;
+  if (t4 > 256) {
+    const bool takes = pl.path == PATH_GEMM ? ring_past_one_round(a, t4) : !nf4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES;
+    return takes ? 4 : 0;
+  }
+  if (dense && a->K > 3072 && a->M > 64) return 0;
+  if (!dense && a->group_size < a->K && !groups32 && a->K >= 8192 && t4 <= 192) return 0;
+  return a->K > (groups32 ? 256 : bits8 || nf4 ? 384 : 512) ? 4 : 0;
 }
 
 // K slices (two and more) in which ring_gemm_kernel takes a call whose plan splits K, with *rt
