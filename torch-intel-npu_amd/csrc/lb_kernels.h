@@ -8,6 +8,8 @@
 //   unpack_kernel, dequant_kernel   bit-exact decode used by tests and by callers that
 //                  want the reference's dequantized fp16 weights on device.
 #pragma once
+#include <type_traits>
+
 #include "lb_common.h"
 
 namespace lb {
@@ -261,21 +263,34 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_kernel(LinearParams p, int 
 }
 
 // Sums split-K partials in a fixed order (deterministic) and applies the epilogue; grid (N / 256, M).  Bound by
-// the latency of its loads, so eight slices' partials are requested before the first is added (one at a time,
-// with a 64-bit division for the row: 24x4096 over 16 slices 6.5 us, now 2.9).
+// the latency of its loads over many slices, so up to eight slices' partials are requested before the first is added
+// (one at a time, with a 64-bit division for the row: 24x4096 over 16 slices 6.5 us, now 2.9), and by issuing them
+// over the two to four of the tiled GEMMs, so never more loads than slices.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(LinearParams p) {
   const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
   if (n >= p.N) return;
   const size_t slice = (size_t)p.M * p.N;
   const float *at = p.partial + (size_t)m * p.N + n;
   float s = 0.0f;
-  for (int sp = 0; sp < p.splits; sp += 8) {
-    float v[8];
+  auto add = [&](auto count) {
+    float v[count.value];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = at[(size_t)min(sp + i, p.splits - 1) * slice];
+    for (int i = 0; i < count.value; ++i) v[i] = at[i * slice];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (sp + i < p.splits) s += v[i];
+    for (int i = 0; i < count.value; ++i) s += v[i];
+    at += count.value * slice;
+  };
+  int left = p.splits;
+  for (; left >= 8; left -= 8) add(std::integral_constant<int, 8>{});
+  switch (left) {  // (uniform)
+    case 1: add(std::integral_constant<int, 1>{}); break;
+    case 2: add(std::integral_constant<int, 2>{}); break;
+    case 3: add(std::integral_constant<int, 3>{}); break;
+    case 4: add(std::integral_constant<int, 4>{}); break;
+    case 5: add(std::integral_constant<int, 5>{}); break;
+    case 6: add(std::integral_constant<int, 6>{}); break;
+    case 7: add(std::integral_constant<int, 7>{}); break;
+    default: break;
   }
   store_output(p, m, n, s);
 }
