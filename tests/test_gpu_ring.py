@@ -55,7 +55,7 @@ def test_ring_fp16_rows(device):
     """fp16 weights (no scales) against a double product, a ragged last stage included."""
     announce('ring fp16')
     rng = np.random.default_rng(3)
-    for m, n, k in ((40, 70, 96), (256, 576, 576), (65, 300, 1536), (100, 2050, 4128), (330, 2700, 3104), (330, 2700, 544)):
+    for m, n, k in ((40, 70, 96), (256, 576, 576), (65, 300, 1536), (100, 2050, 4128), (330, 2700, 3104), (330, 2700, 544), (50, 1000, 6400)):
         x = rng.standard_normal((m, k)).astype(np.float16)
         w = (rng.standard_normal((n, k)) * 0.02).astype(np.float16)
         y = lowbit_hip.linear(to_dev(x, device), to_dev(w, device), None, format='fp16', N=n, K=k, group_size=k)

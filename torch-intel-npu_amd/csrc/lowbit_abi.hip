@@ -441,11 +441,11 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 // tiles in groups 266x2048x8192 31.4 -> 35.3; NF4 in groups of 32 already from 3072 codes on, 462x76x4096 12.6 -> 18.2)
 // and, for NF4, whose table reads load LDS, past 4096 codes (300x2048x8192 32.3 -> 38.6).  So does fp16, whose weights
 // gemm4_kernel's larger tiles read fewer times, past 3072 codes in 64-row tiles (513x1424x12096 43.1 -> 68.6; but
-// 801x769x2176 18.6 -> 16.8, one row of tiles 62x14336x4096 32.3 -> 25.6) and past 4096 in 32-row ones over many columns
-// whose tiles of one column meet on different XCDs (55x6574x9152 29.8 -> 37.0; 178x2048x8192 22.4 -> 19.4,
-// 480x657x5952 23.3 -> 19.6).  Full rounds of 64-row tiles need rows that outlast filling the ring (INT4 186x4546x512
-// 6.9 -> 7.7, 212x2944x704 9.4 -> 7.0; INT8 and NF4 682x1166x256 6.2 -> 7.0, 562x946x448 7.2 -> 6.9; in groups of 32,
-// which gemm4_kernel scales code by code, 310x3089x256 6.1 -> 7.3, 474x1439x288 7.4 -> 7.0).
+// 801x769x2176 18.6 -> 16.8, one row of tiles 62x14336x4096 32.3 -> 25.6) and past 4096 in smaller ones over many
+// columns whose tiles of one column meet on different XCDs (45x3230x12768 25.1 -> 38.4, 55x6574x9152 29.8 -> 37.0;
+// 178x2048x8192 22.4 -> 19.4, 480x657x5952 23.3 -> 19.6).  Full rounds of 64-row tiles need rows that outlast filling
+// the ring (INT4 186x4546x512 6.9 -> 7.7, 212x2944x704 9.4 -> 7.0; INT8 and NF4 682x1166x256 6.2 -> 7.0, 562x946x448
+// 7.2 -> 6.9; in groups of 32, which gemm4_kernel scales code by code, 310x3089x256 6.1 -> 7.3, 474x1439x288 7.4 -> 7.0).
 // Of the calls of up to 32 rows: 17 and more over short rows or enough columns (wide_rows / tile_rows -> ring:
 // INT8 24x14336x4096 24.4 -> 17.9, 32x8192x2048 13.0 -> 8.6, 17x1536x576 4.8 -> 4.1, INT4 32x11008x4096 20.6 -> 13.4,
 // 32x576x1536 7.5 -> 6.0, NF4 32x8192x3072 16.1 -> 10.9; but 24x1024x4096 8.8 -> 9.9, NF4 32x4096x4096 12.5 -> 14.3),
@@ -516,9 +516,9 @@ int ring_rt(const lb_linear_args *a, const Plan &pl) {
     if (a->K > 4096 && t1 <= 128) return 0;
     if (nf4 && groups32 && a->K >= 3072 && a->K % 64 == 0 && t1 <= 128 && a->rank == 0) return 0;
   }
+  if (a->rank == 0 && t2 <= 256 && dense && a->K > 4096 && cols > 12 && cols % 8 != 0) return 0;
   if (t1 <= 256) return 1;
-  if (a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
-  if (t2 <= 256) return dense && a->K > 4096 && cols > 24 && cols % 8 != 0 ? 0 : 2;
+  if (t2 <= 256 || a->rank > 0) return t2 <= LB_RING_MAX_TILES ? 2 : 0;
   if (t4 > 256) {
     const bool takes = pl.path == PATH_GEMM ? ring_past_one_round(a, t4) : !nf4 && a->K >= 2048 && t4 <= LB_RING_MAX_TILES;
     return takes ? 4 : 0;
