@@ -19,9 +19,15 @@ from torch_npu_smollm_io import FrozenSmolIO
 pytestmark = pytest.mark.gpu
 
 
-def layer(mode, rank=0, capacity=160, protected=(), seed=3):
+# Deviations of the weights: small ones leave a row nearly its residual; PEAKED ones give attention over many keys a
+# few large probabilities and more than half of the output.
+PEAKED = {'self_attn.q_proj.weight': 0.07, 'self_attn.k_proj.weight': 0.07, 'self_attn.v_proj.weight': 0.08,
+          'self_attn.o_proj.weight': 0.08}
+
+
+def layer(mode, rank=0, capacity=160, protected=(), seed=3, deviations={}):
     g = torch.Generator().manual_seed(seed)
-    weights = {n: (torch.randn(s, generator=g) * 0.02 if len(s) == 2 else 1 + 0.1 * torch.randn(s, generator=g)).half()
+    weights = {n: (torch.randn(s, generator=g) * deviations.get(n, 0.02) if len(s) == 2 else 1 + 0.1 * torch.randn(s, generator=g)).half()
                for n, s in _SHAPES.items()}
     packed = corrections = None
     if rank:
@@ -65,6 +71,31 @@ def test_layer_rows_prefill_and_decode(device, mode, rank, batch, seq):
         again, _ = lay.decode(x[:, seq:seq + 1].to(device), first)
         assert torch.equal(again, outs[0])
         assert rel(lay(x.to(device)), want) <= 1e-2
+
+
+@pytest.mark.parametrize('mode,rank,batch,seq', [('w8a16', 4, 1, 33), ('fp16', 0, 2, 130), ('w8a16', 32, 1, 257),
+                                                 ('fp16', 0, 3, 288), ('w4a16', 0, 1, 513), ('nf4a16', 0, 2, 700),
+                                                 ('w8a16', 8, 1, 1025), ('w8a16', 0, 1, 2016)])
+def test_layer_rows_attention_of_few_large_weights(device, mode, rank, batch, seq):
+    """Past 256 keys attention takes further rounds of score tiles, recomputed exponentials and reloaded values: whole
+    prefills, the same rows in two calls (the second at a start of its own), and a decode at the last slot.  Without
+    their last 32 keys the last rows would move by ten times the bar and more."""
+    announce('layer rows long', mode, rank, batch, seq)
+    lay = layer(mode, rank, capacity=2016, deviations=PEAKED)
+    x = torch.randn(batch, seq, 576, generator=torch.Generator().manual_seed(seq)).half()
+    want, trace = lay.reference_cpu(x)
+    dev, rows = x.to(device), lay._dev(device)['rows']
+    with torch.no_grad():
+        out, cache = lay.prefill(dev)
+        assert rel(out, want) <= 1e-2 and rel(out[:, -17:], want[:, -17:]) <= 1e-2
+        assert rel(cache.keys[:, :, :seq], trace['keys']) <= 1e-2 and rel(cache.values[:, :, :seq], trace['values']) <= 1e-2
+        keys, values = torch.zeros(2, batch, 3, 2016, 64, dtype=torch.float16, device=device)
+        first = seq // 2 + 3
+        parts = [rows.run(dev[:, :first], keys, values, 0), rows.run(dev[:, first:], keys, values, first)]
+        assert rel(torch.cat(parts, 1), want) <= 1e-2 and rel(keys, cache.keys.cpu()) <= 1e-2
+        _, short = lay.prefill(dev[:, :-1])
+        last, _ = lay.decode(dev[:, -1:], short)
+        assert rel(last, want[:, -1:]) <= 1e-2
 
 
 def test_layer_rows_do_not_read_past_the_position(device):
@@ -172,7 +203,7 @@ def test_one_row_over_a_long_cache(device):
 
 
 def test_batches_past_the_launch_limits_are_staged(device):
-    """65536 sequences (one past a grid's z range) still run: their first rows are those of a small batch."""
+    """65536 sequences (one past a grid's z range) still run, and 349184 rows within the limits: the last are a small batch's."""
     announce('layer rows limits')
     lay = layer('w4a16', capacity=8)
     rows = lay._dev(device)['rows']
@@ -181,3 +212,7 @@ def test_batches_past_the_launch_limits_are_staged(device):
     with torch.no_grad():
         want = lay(x)
         assert rel(lay(x.repeat(1024, 1, 1))[-64:], want.cpu()) <= 1e-2
+        x = torch.randn(64, 8, 576, generator=torch.Generator().manual_seed(5)).half().to(device)
+        assert rows.fits(64 * 682, 8) and not rows.fits(64 * 683, 8)
+        want = lay(x)
+        assert rel(lay(x.repeat(682, 1, 1))[-64:], want.cpu()) <= 1e-2   # 349184 rows in lb_layer_rows
