@@ -354,8 +354,10 @@ def decode_leg(device, steps, cpu_steps):
     ids = smollm_random.prompt(seed=0, length=256).to(device)
     out = {}
     with torch.no_grad():
-        for _ in range(2):  # warm (device copies of weights, allocator)
+        for _ in range(2):  # warm all that is timed below (device copies of weights, allocator, first launches)
             h, caches = stack.prefill(io.embed_tokens(ids))
+            first = int(io.logits(h[:, -1:])[0, 0].float().argmax())
+            stack.decode(io.embed_tokens(torch.tensor([[first]], device=device)), caches)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         h, caches = stack.prefill(io.embed_tokens(ids))
