@@ -172,6 +172,21 @@ def test_copies_of_used_modules(device):
             assert torch.equal(copy.deepcopy(a)(arg), want) and torch.equal(a(arg.contiguous()), want)
 
 
+def test_padded_factors_are_complete_for_every_stream(device, monkeypatch):
+    """Factors of odd ranks are padded on the stream of the first call, whose work the constructor waits for."""
+    announce('padded factors')
+    waited = []
+    monkeypatch.setattr(torch.cuda.Stream, 'synchronize', lambda self: waited.append(torch.cuda.synchronize(device)))
+    for rank, waits in ((8, 0), (4, 1)):
+        waited.clear()
+        lay = layer('w8a16', rank)
+        lay._dev(device)
+        assert len(waited) == waits
+        x = torch.randn(1, 3, 576, generator=torch.Generator().manual_seed(8)).half()
+        with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream(device)):
+            assert rel(lay(x.to(device)), lay.reference_cpu(x)[0]) <= 1e-2
+
+
 def test_layer_rows_refuses(device):
     announce('layer rows refuses')
     lay = layer('w4a16', capacity=8)

@@ -939,6 +939,7 @@ class LayerRows:
         keep = [_row(norm1, 'norm1', hidden), _row(norm2, 'norm2', hidden), _row(cos, 'cos', a.capacity * 64),
                 _row(sin, 'sin', a.capacity * 64)]
         a.norm1, a.norm2, a.cos, a.sin = (_ptr(t) for t in keep)
+        padded = False
         for q, pr in zip(a.proj, projections):
             q.format, q.group_size, q.N, q.K = FORMATS[pr['format']], pr['group'], pr['N'], pr['K']
             q.codes, q.scales = _ptr(pr['codes']), _ptr(pr.get('scales'))
@@ -949,9 +950,12 @@ class LayerRows:
                 if rank != down.shape[0] or up.stride(-1) != 1 or up.stride(0) % 8:  # whole eights: zero ranks add nothing
                     down = torch.cat((down, down.new_zeros(rank - down.shape[0], down.shape[1])))
                     up = torch.cat((up, up.new_zeros(up.shape[0], rank - up.shape[1])), 1)
+                    padded = True
                 down = down.contiguous()
                 q.rank, q.down, q.up, q.up_ld = rank, _ptr(down), _ptr(up), up.stride(0)
                 keep += [down, up]
+        if padded:  # written on this stream, read on any
+            torch.cuda.current_stream(norm1.device).synchronize()
         self._template, self._keep, self._device = a, keep, norm1.device
         self._fn = library().lb_layer_rows
 
