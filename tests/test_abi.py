@@ -626,7 +626,9 @@ calls = [('lb_linear', lambda: lib.lb_linear(ctypes.byref(a), None)),
          ('lb_decode_attention', lambda: lib.lb_decode_attention(ctypes.byref(lowbit_hip.DecodeAttentionArgs()), None)),
          ('lb_argmax_next', lambda: lib.lb_argmax_next(0x1, 16, 0x2, 8, 0x3, 0x4, 0x5, 0x6, 4, None)),
          ('lb_head_next', lambda: lib.lb_head_next(ctypes.byref(lowbit_hip.FusedLinearArgs()), 0x1, 0x2, 0x3, 0x4, 0x5,
-                                                   4, None))]
+                                                   4, None)),
+         ('lb_rms_rows', lambda: lib.lb_rms_rows(0x10000, 0x20000, 0x30000, 1, 64, 1e-5, None)),
+         ('lb_layer_rows', lambda: lib.lb_layer_rows(ctypes.byref(lowbit_hip.LayerRowsArgs()), None))]
 for name, call in calls:
     assert call() == lowbit_hip.DEVICE_FAILED, name
     message = lib.lb_last_error().decode()
