@@ -452,8 +452,9 @@ int wide_slices(int fmt, int64_t N, int64_t K) {
 // long rows that wide_rows_kernel does not cut (a prime number of its chunks: INT8 17x4096x11008 136 -> 25), 9 to 16
 // over large weights in one round (INT4 16x11008x4096 16.7 -> 11.9, NF4 12x11008x4096 20.7 -> 15.1; INT4
 // 16x8192x3072 8.7 -> 9.1) or where a second one is over half full and tile_rows_kernel does not take them (9x19834x3712
-// 22.3 -> 31.2, 11x28779x3712 35.6 -> 31.1; INT8 11x25759x2048 16.6 -> 20.4), and every call
-// with a correction (no z launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7).
+// 22.3 -> 31.2, 11x28779x3712 35.6 -> 31.1; INT8 11x25759x2048 16.6 -> 20.4), and calls
+// with a correction (no z launch and no second pass: rank 32 W8 8x576x576 16.9 -> 4.9, 24x4096x4096 37.6 -> 14.7,
+// 1024x1088x576, 544 tiles, 25.1 -> 15.1; more tiles keep the three launches, 2000x576x576 25.1).
 // Not where wide_rows_kernel cuts 4-bit rows into few slices, nor where 17 rows and more suit tile_rows_kernel: one
 // round of its pairs of tiles (INT4 19x7588x640 4.6 -> 6.0, 17x7939x960 4.9 -> 6.8; 23x5898x704 9.6 -> 5.5 before the
 // pairs fill it), and the lengths it stages exactly, 1024 over few columns (INT4 23x1878 5.3 -> 5.8, but 28x1984x896

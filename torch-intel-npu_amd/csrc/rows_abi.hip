@@ -42,7 +42,10 @@ void launch_mode(const RingParams &p, int format, bool ranked, int rt, int tiles
   }
 }
 
-// Rows per workgroup (in sixteens): the smallest tile that leaves one round of 256 workgroups (lb_linear's rule).
+// Rows per workgroup (in sixteens): the smallest tile that leaves one round of 256 workgroups, past one round the largest
+// there is (RoPE, the cache's append, SiLU and the residual are part of the launch, which gemm4_kernel's larger tiles
+// have no form of).  A layer of 8 x 256 rows takes 146 us with W8 and rank 32, 94 with INT4, 64 x 256 rows 905 and 506,
+// one prompt of 2000 rows 208 and 156; lb_linear per projection between torch operations 538, 438, 1528, 1131, 847, 687.
 int rows_rt(int64_t M, int64_t tiles, bool ranked) {
   if ((M + 15) / 16 * tiles <= 256) return 1;
   if ((M + 31) / 32 * tiles <= 256 || ranked) return 2;
