@@ -458,7 +458,7 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float gate = (float)v[e];
-        const f16 act = (f16)(gate / (1.0f + expf(-gate)));
+        const f16 act = (f16)(gate / (1.0f + __expf(-gate)));
         v[e] = (f16)((float)act * (float)up[e]);
       }
     }
