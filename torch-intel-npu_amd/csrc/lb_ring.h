@@ -455,6 +455,8 @@ __global__ __launch_bounds__(kRingThreads) void ring_gemm_kernel(RingParams p) {
     h8 v = *reinterpret_cast<const h8 *>(out_at(r, c));
     if constexpr (PAIR) {
       const h8 up = *reinterpret_cast<const h8 *>(out_at(r, 32 + c));
+      // __expf: over all finite fp16 gates the rounded SiLU is off by rms 1.71271e-4 of its value, as with expf (3 and 1
+      // of 63488 differ from the rounded 64-bit value); expf takes 0.6 us more a launch (256 rows, 1536 columns).
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float gate = (float)v[e];

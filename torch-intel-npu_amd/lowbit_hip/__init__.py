@@ -906,7 +906,7 @@ class PreparedStack(_Prepared):
 # ---------------------------------------------------------------- several token rows
 def _aligned(t):
     """t, contiguous and at a 16-byte address (a contiguous view may begin at any element)."""
-    t = t.detach().contiguous()
+    t = t.contiguous()
     return t.clone() if t.data_ptr() % 16 else t
 
 
