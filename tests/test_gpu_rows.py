@@ -123,6 +123,7 @@ def test_layer_rows_and_protected_projections(device, protected, rows):
     want, _ = lay.reference_cpu(x)
     with torch.no_grad():
         assert rel(lay(x.to(device)), want) <= 1e-2
+        assert torch.equal(lay._full(x.to(device), None), lay.prefill(x.to(device))[0])   # forward keeps no cache
 
 
 @pytest.mark.parametrize('rows,width', [(1, 576), (5, 8), (3, 4096), (257, 520)])

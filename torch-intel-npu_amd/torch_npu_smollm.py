@@ -348,10 +348,12 @@ class FrozenSmolLayer(torch.nn.Module):
 
     def _full(self, x, both):
         """Causal full-sequence layer on device; keys and values go to slots 0 .. S - 1 of
-        both [2, B, 3, slots, 64]."""
+        both [2, B, 3, slots, 64] (None: to nobody)."""
         state = self._dev(x.device)
         b, s, d = x.shape
         if 'rows' in state and state['rows'].fits(b, s):
+            if both is None:  # lb_layer_rows attends over them
+                both = torch.empty((2, b, KV_HEADS, s, HEAD_DIM), dtype=torch.float16, device=x.device)
             return state['rows'].run(x, both[0], both[1], 0)
         n1 = self._norm(x, state['norm1']).view(b * s, d)
         q = self._linear(state, n1, 'self_attn.q_proj.weight').view(b, s, HEADS, HEAD_DIM).transpose(1, 2)
@@ -363,13 +365,14 @@ class FrozenSmolLayer(torch.nn.Module):
         att = self._attend(q, k, v, mask).transpose(1, 2).reshape(b * s, d)
         delta = self._linear(state, att, 'self_attn.o_proj.weight').view(b, s, d)
         value = (x + delta).half()
-        both[0, :, :, :s] = k
-        both[1, :, :, :s] = v
+        if both is not None:
+            both[0, :, :, :s] = k
+            both[1, :, :, :s] = v
         return self._mlp(state, value)
 
     def forward(self, x):
-        b, s, _ = self._validate_input(x)
-        return self._full(x, torch.empty((2, b, KV_HEADS, s, HEAD_DIM), dtype=torch.float16, device=x.device))
+        self._validate_input(x)
+        return self._full(x, None)
 
     def prefill(self, x):
         """Full prefix; returns the output and a KV snapshot (reference :506-523)."""
